@@ -1601,6 +1601,28 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype = torch.flo
     return out
 
 
+def gemm_tn_f32_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether gemm_tn_f32 takes these operands: F32 2-D CUDA tensors with
+    equal row counts and unit column stride (any widths and row strides)."""
+    return (a.is_cuda and b.is_cuda and a.dim() == 2 and b.dim() == 2 and a.dtype == torch.float32
+            and b.dtype == torch.float32 and a.shape[0] == b.shape[0] and a.stride(1) == 1 and b.stride(1) == 1)
+
+
+def gemm_tn_f32(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a^T @ b for F32 a [K, M], b [K, N] (split over K, deterministic)."""
+    if not gemm_tn_f32_supported(a, b):
+        raise ValueError("gemm_tn_f32: unsupported operands (see gemm_tn_f32_supported)")
+    L.require_device("gemm_tn_f32", a.device, b)
+    K, M = a.shape
+    N = b.shape[1]
+    out = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    wsb = int(L.load().grws_gemm_tn_f32_workspace_bytes(K, M, N))
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=a.device)
+    L.call("grws_gemm_tn_f32", L.ptr(a), a.stride(0), L.ptr(b), b.stride(0), K, M, N, L.ptr(out), N, L.ptr(ws), wsb,
+           L.stream_of(a.device))
+    return out
+
+
 # ---------------------------------------------------------------------------
 # halo-aware subgraph repack (sampler/sampler.py:420-690)
 # ---------------------------------------------------------------------------

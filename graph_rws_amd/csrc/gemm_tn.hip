@@ -159,6 +159,130 @@ __global__ __launch_bounds__(256) void gemm_tn_partial_kernel(const uint16_t* __
         }
 }
 
+// The same product for f32 operands on v_mfma_f32_16x16x4_f32 (grws_gemm_tn_f32).
+//
+// Bound by the f32 matrix rate: 157 TFLOP/s at most, so 71 us for K =
+// 169,343, 128 x 256 (the operands' 260 MB take 52 us at 5 TB/s).  Measured:
+// 116 us with the reduction (96 TFLOP/s); the library's product takes 440 us
+// (too few work-groups over K).  On 64 x 64 columns 28 us (342), 16 x 7
+// 17 us (147).  Each
+// wave owns 16 TA x 16 TB outputs, 2 x 2 waves a work-group; the smallest
+// TA, TB of {1, 2, 4} that cover M and N are taken, so a 7-column class
+// layer does not pay for 128 columns.  An operand of the MFMA is one 4-byte
+// LDS read a lane (row 4 k + lane / 16, 16 consecutive columns; the pitch of
+// 16 mod 64 words puts the four rows on different banks): TA + TB reads for
+// TA TB MFMAs of 32 cycles, so plain reads suffice where the 16-bit kernel
+// needs the transposing ones.
+constexpr int kStepF = 32;  // K rows per LDS stage
+
+template <int TA, int TB, bool VEC>
+__global__ __launch_bounds__(256) void gemm_tn_f32_partial_kernel(const float* __restrict__ A, int64_t lda,
+                                                                  const float* __restrict__ B, int64_t ldb,
+                                                                  int64_t K, int M, int N, int64_t kc,
+                                                                  int64_t nchunks, float* __restrict__ partials) {
+    constexpr int CA = 32 * TA, CB = 32 * TB;  // the work-group's columns of A and B
+    constexpr int PA = CA % 64 ? CA + 48 : CA + 16, PB = CB % 64 ? CB + 48 : CB + 16;  // 16 mod 64
+    __shared__ __attribute__((aligned(16))) float sA[2][kStepF * PA];
+    __shared__ __attribute__((aligned(16))) float sB[2][kStepF * PB];
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6;
+    const int lane = tid & 63;
+    // chunks dealt to XCDs as in gemm_tn_partial_kernel
+    const int tiles_m = (M + CA - 1) / CA;
+    const int tiles = tiles_m * ((N + CB - 1) / CB);
+    const int64_t blk = blockIdx.x;
+    const int64_t slot = blk >> 3;
+    const int t = (int)(slot % tiles);
+    const int64_t chunk = (slot / tiles) * 8 + (blk & 7);
+    if (chunk >= nchunks) return;  // uniform over the work-group
+    const int i0 = (t % tiles_m) * CA;
+    const int j0 = (t / tiles_m) * CB;
+    const int64_t kb = chunk * kc;
+    const int64_t ke = kb + kc < K ? kb + kc : K;
+    const int wm = (wave & 1) * 16 * TA;
+    const int wn = (wave >> 1) * 16 * TB;
+    const int fr = lane & 15;
+    const int fg = lane >> 4;
+
+    float4_t acc[TA][TB];
+#pragma unroll
+    for (int a = 0; a < TA; ++a)
+#pragma unroll
+        for (int b = 0; b < TB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    // 32 rows x 32 TA columns = TA loads of 4 elements a thread; VEC:
+    // both operands' rows are whole 16-byte vectors, else four loads each
+    // (a flag read at run time instead cost the aligned form 114 -> 155 us)
+    float4_t ra[TA], rb[TB];
+    auto load4 = [](const float* p, int left) {
+        float4_t v{0.f, 0.f, 0.f, 0.f};
+        if constexpr (VEC) {
+            if (left > 0) v = *reinterpret_cast<const float4_t*>(p);
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                if (x < left) v[x] = p[x];
+        }
+        return v;
+    };
+    auto fetch = [&](int64_t k0) {
+#pragma unroll
+        for (int q = 0; q < TA; ++q) {
+            const int e = (tid + 256 * q) * 4;
+            const int r = e / CA, c = e % CA;
+            ra[q] = load4(A + (k0 + r) * lda + i0 + c, k0 + r < ke ? M - i0 - c : 0);
+        }
+#pragma unroll
+        for (int q = 0; q < TB; ++q) {
+            const int e = (tid + 256 * q) * 4;
+            const int r = e / CB, c = e % CB;
+            rb[q] = load4(B + (k0 + r) * ldb + j0 + c, k0 + r < ke ? N - j0 - c : 0);
+        }
+    };
+    int buf = 0;
+    if (kb < ke) fetch(kb);
+    for (int64_t k0 = kb; k0 < ke; k0 += kStepF) {
+#pragma unroll
+        for (int q = 0; q < TA; ++q) {
+            const int e = (tid + 256 * q) * 4;
+            *reinterpret_cast<float4_t*>(&sA[buf][(e / CA) * PA + e % CA]) = ra[q];
+        }
+#pragma unroll
+        for (int q = 0; q < TB; ++q) {
+            const int e = (tid + 256 * q) * 4;
+            *reinterpret_cast<float4_t*>(&sB[buf][(e / CB) * PB + e % CB]) = rb[q];
+        }
+        __syncthreads();  // the stage is written; the other stage's readers are done
+        if (k0 + kStepF < ke) fetch(k0 + kStepF);
+#pragma unroll
+        for (int ks = 0; ks < kStepF; ks += 4) {
+            float af[TA], bf[TB];
+#pragma unroll
+            for (int a = 0; a < TA; ++a) af[a] = sA[buf][(ks + fg) * PA + wm + 16 * a + fr];
+#pragma unroll
+            for (int b = 0; b < TB; ++b) bf[b] = sB[buf][(ks + fg) * PB + wn + 16 * b + fr];
+#pragma unroll
+            for (int a = 0; a < TA; ++a)
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[a], bf[b], acc[a][b], 0, 0, 0);
+        }
+        buf ^= 1;
+    }
+    float* P = partials + chunk * (int64_t)M * N;
+#pragma unroll
+    for (int a = 0; a < TA; ++a)
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const int j = j0 + wn + 16 * b + fr;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = i0 + wm + 16 * a + 4 * fg + e;
+                if (i < M && j < N) P[(int64_t)i * N + j] = acc[a][b][e];
+            }
+        }
+}
+
 // C[i][j] = sum over chunks.  A work-group of 16 waves covers 64
 // consecutive outputs; wave w adds chunks w, w+16, ... in order (coalesced
 // 256-byte rows), then wave 0 adds the 16 wave sums in order: a fixed order
@@ -210,10 +334,96 @@ int64_t chunks_for(int64_t K, int64_t M, int64_t N) {
     return n < 1 ? 1 : n;
 }
 
+// f32: 16-column blocks a wave takes of an operand `cols` wide (two waves
+// side by side), and the K-chunks.  Every work-group holds a matrix core for
+// the whole launch, so the chunks are counted to fill the 256 CUs evenly,
+// kBlocksF work-groups in all, of at least kSmallChunkRows rows.
+constexpr int64_t kBlocksF = 512;
+
+int f32_blocks(int64_t cols) { return cols <= 32 ? 1 : cols <= 64 ? 2 : 4; }
+
+struct F32Shape {
+    int ta, tb;
+    int64_t tiles, chunks;
+};
+
+F32Shape f32_shape(int64_t K, int64_t M, int64_t N) {
+    F32Shape s;
+    s.ta = f32_blocks(M);
+    s.tb = f32_blocks(N);
+    s.tiles = ((M + 32 * s.ta - 1) / (32 * s.ta)) * ((N + 32 * s.tb - 1) / (32 * s.tb));
+    int64_t n = s.tiles > 0 ? kBlocksF / s.tiles / 8 * 8 : 1;
+    const int64_t most = (K + kSmallChunkRows - 1) / kSmallChunkRows;
+    if (n < 8) n = 8;
+    if (n > most) n = most;
+    s.chunks = n < 1 ? 1 : n;
+    return s;
+}
+
+template <int TA, int TB>
+void launch_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int64_t K, int64_t M, int64_t N, int64_t kc,
+                int64_t chunks, unsigned blocks, float* partials, hipStream_t stream) {
+    const bool vec = M % 4 == 0 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && N % 4 == 0 &&
+                     ldb % 4 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+    if (vec)
+        hipLaunchKernelGGL((gemm_tn_f32_partial_kernel<TA, TB, true>), dim3(blocks), dim3(256), 0, stream, a, lda, b,
+                           ldb, K, (int)M, (int)N, kc, chunks, partials);
+    else
+        hipLaunchKernelGGL((gemm_tn_f32_partial_kernel<TA, TB, false>), dim3(blocks), dim3(256), 0, stream, a, lda, b,
+                           ldb, K, (int)M, (int)N, kc, chunks, partials);
+}
+
 }  // namespace
 }  // namespace grws
 
 using namespace grws;
+
+extern "C" size_t grws_gemm_tn_f32_workspace_bytes(int64_t K, int64_t M, int64_t N) {
+    if (K < 0 || M < 0 || N < 0) return 0;
+    return (size_t)f32_shape(K, M, N).chunks * (size_t)M * (size_t)N * sizeof(float);
+}
+
+extern "C" int grws_gemm_tn_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int64_t K, int64_t M,
+                                int64_t N, float* c, int64_t ldc, void* workspace, size_t workspace_bytes,
+                                void* stream_) {
+    clear_error();
+    hipStream_t stream = as_stream(stream_);
+    GRWS_CHECK_ARG(K >= 0 && M >= 0 && N >= 0, "gemm_tn_f32: negative size");
+    GRWS_CHECK_ARG(M <= 65536 && N <= 65536, "gemm_tn_f32: M and N must be at most 65536");
+    GRWS_CHECK_ARG(lda >= M && ldb >= N && ldc >= N, "gemm_tn_f32: leading dimensions too small");
+    if (M == 0 || N == 0) return GRWS_OK;
+    GRWS_CHECK_ARG(c != nullptr, "gemm_tn_f32: null output");
+    const F32Shape sh = f32_shape(K, M, N);
+    int64_t chunks = 0;  // K == 0: the reduction over no chunks writes zeros
+    if (K > 0) {
+        GRWS_CHECK_ARG(a && b, "gemm_tn_f32: null input");
+        const size_t need = (size_t)sh.chunks * (size_t)M * (size_t)N * sizeof(float);
+        if (!workspace || workspace_bytes < need)
+            return set_error(GRWS_E_CAPACITY, "gemm_tn_f32: workspace too small (%zu < %zu)", workspace_bytes, need);
+        const int64_t kc = ((K + sh.chunks - 1) / sh.chunks + kStepF - 1) / kStepF * kStepF;
+        chunks = (K + kc - 1) / kc;
+        const int64_t blocks = (chunks + 7) / 8 * 8 * sh.tiles;
+        GRWS_CHECK_ARG(blocks <= INT32_MAX, "gemm_tn_f32: too many work-groups");
+        float* P = static_cast<float*>(workspace);
+        const unsigned g = (unsigned)blocks;
+        switch (sh.ta * 8 + sh.tb) {
+            case 9: launch_f32<1, 1>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 10: launch_f32<1, 2>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 12: launch_f32<1, 4>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 17: launch_f32<2, 1>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 18: launch_f32<2, 2>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 20: launch_f32<2, 4>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 33: launch_f32<4, 1>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            case 34: launch_f32<4, 2>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+            default: launch_f32<4, 4>(a, lda, b, ldb, K, M, N, kc, chunks, g, P, stream); break;
+        }
+        GRWS_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(gemm_tn_reduce_kernel<GRWS_F32>, dim3((unsigned)((M * N + 63) / 64)), dim3(1024), 0, stream,
+                       static_cast<const float*>(workspace), chunks, (int)M, (int)N, c, ldc);
+    GRWS_LAUNCH_CHECK();
+    return GRWS_OK;
+}
 
 extern "C" size_t grws_gemm_tn_workspace_bytes(int64_t K, int64_t M, int64_t N) {
     if (K < 0 || M < 0 || N < 0) return 0;

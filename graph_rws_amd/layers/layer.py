@@ -37,6 +37,13 @@ FUSED_SELF = True
 PAD_AGGREGATE = True
 
 
+# Rows from which an f32 weight gradient takes the split-K kernel.  Measured
+# (us, library / kernel): 128 x 256 at 4,096 rows 26 / 32, at 16,384 rows
+# 99 / 31, at 169,343 rows 440 / 116; 608 x 256 at 4,096 rows 27 / 41, at
+# 16,384 rows 107 / 69; 1433 x 16 at 4,096 rows 20 / 21, at 16,384 55 / 38.
+F32_TN_ROWS = 16384
+
+
 def _spmm_timed(graph, x: torch.Tensor, residual: torch.Tensor = None):
     """graph.spmm with the reference's (output, ms) convention (bind.cpp:124-130)."""
     if not _ops.TIMING:
@@ -63,9 +70,14 @@ def _autocast_operand(x: torch.Tensor) -> torch.Tensor:
 def _weight_grad(x: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     """x^T @ g: the split-K gfx950 kernel for tall f16/bf16 operands (the
     library GEMM leaves most of the chip idle on this shape), torch
-    otherwise.  float32 result from the kernel."""
+    otherwise.  float32 result from the kernel.  Tall f32 operands take the
+    f32 kernel, except where autocast would multiply them in 16 bits and in
+    a backward that is itself recorded (create_graph)."""
     if x.shape[0] >= 4096 and _ops.gemm_tn_supported(x, g):
         return _ops.gemm_tn(x, g, out_dtype=torch.float32)
+    if (x.shape[0] >= F32_TN_ROWS and _ops.gemm_tn_f32_supported(x, g) and not torch.is_grad_enabled()
+            and not torch.is_autocast_enabled("cuda")):
+        return _ops.gemm_tn_f32(x, g)
     return torch.matmul(x.t(), g)
 
 

@@ -4,7 +4,7 @@ the same f16/bf16 inputs.  Bound: |C - C64| <= 1e-4 * (|A|^T |B|) elementwise
 import pytest
 import torch
 
-from graph_rws_amd.core.ops import gemm_tn, gemm_tn_supported
+from graph_rws_amd.core.ops import gemm_tn, gemm_tn_f32, gemm_tn_supported
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +90,26 @@ def test_graphconv_autocast_backward_uses_split_k(cuda_device):
         assert got.dtype == torch.float32
         d = float((got.double().cpu() - want).abs().max())
         assert d <= 2e-2 * float(want.abs().max()), d
+
+
+@pytest.mark.parametrize("K,M,N", [(0, 8, 16), (1, 4, 4), (31, 32, 36), (255, 33, 64), (257, 65, 7), (4097, 64, 129),
+                                   (9000, 1433, 16), (100003, 128, 256), (65536, 200, 41)])
+def test_gemm_tn_f32_matches_float64(cuda_device, K, M, N):
+    """Edges of the 32/64/128-column tiles, ragged widths and K
+    remainders.  Bound: a chunk of k rows summed in f32 in order, then the
+    chunks' partials: (k + chunks) * 2^-24 of |A|^T |B|; chunks have at most
+    max(256, K tiles / 512) + 32 rows, under 8,192 here."""
+    g = torch.Generator(device=cuda_device).manual_seed(K + M + N)
+    A = torch.randn(K, M, generator=g, device=cuda_device)
+    B = torch.randn(K, N, generator=g, device=cuda_device)
+    C = gemm_tn_f32(A, B)
+    assert C.shape == (M, N) and C.dtype == torch.float32
+    ref = A.double().t() @ B.double()
+    bound = A.double().abs().t() @ B.double().abs()
+    assert bool(((C.double() - ref).abs() <= (8192 + 512) * 2.0 ** -24 * bound + 1e-30).all())
+    assert torch.equal(C, gemm_tn_f32(A, B))  # deterministic
+    wide = torch.full((K, N + 9), float("nan"), device=cuda_device)
+    wide[:, :N] = B  # a column view of a wider buffer: its padding must not reach the result
+    assert torch.equal(C, gemm_tn_f32(A, wide[:, :N]))
+    wide[:, 1:N + 1] = B  # a misaligned start
+    assert torch.equal(C, gemm_tn_f32(A, wide[:, 1:N + 1]))

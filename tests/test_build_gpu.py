@@ -581,3 +581,21 @@ def test_build_c2_full_size(cuda_device):
     _eq(hw, ow)
     _eq(hc, oc)
     _eq(hv, ov)
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 1, 1 << 20, (1 << 20) + 8191, (1 << 21) + 1])
+@pytest.mark.parametrize("spread", ["one", "few", "all"])
+def test_large_sort_tiles_are_stable(cuda_device, n, spread):
+    """The 8,192-key tiles of the large sort (2^20 keys and more) at their
+    edges: one digit for every key, a few, and all; the weights are the input
+    positions, so an unstable place or a lost key shows."""
+    print(f"case large sort n={n} {spread}", flush=True)
+    rows = {"one": 1, "few": 5, "all": 70000}[spread]
+    g = torch.Generator(device=cuda_device).manual_seed(n)
+    src = torch.randint(0, rows, (n,), generator=g, device=cuda_device, dtype=torch.int32)
+    dst = torch.randint(0, 3 if spread != "all" else 300, (n,), generator=g, device=cuda_device, dtype=torch.int32)
+    w = torch.arange(n, device=cuda_device, dtype=torch.float32)  # exact below 2^24
+    _, rp, ci, va = builder.coo_to_csr_device(rows, 300, src, dst, w)
+    perm = torch.sort(src.long() * 300 + dst.long(), stable=True).indices
+    assert torch.equal(ci, dst[perm]) and torch.equal(va, w[perm])
+    assert torch.equal(rp[1:] - rp[:-1], torch.bincount(src.long(), minlength=rows))

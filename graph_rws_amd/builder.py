@@ -63,12 +63,17 @@ def _build(row_ptr, rows, cols, values, nnz: int, num_rows: int, num_cols: int, 
     L.call("grws_bcsr_build_count", L.ptr(row_ptr), L.ptr(rows), L.ptr(cols), L.ptr(values), nnz,
            num_rows, num_cols, tile_cols, int(transpose), L.ptr(win), L.ptr(ws), wsb,
            ctypes.byref(T), stream)
-    T = T.value
-    out_cols = torch.empty(T * tile_cols, dtype=torch.int32, device=dev)
-    out_vals = torch.empty(T * 16 * tile_cols, dtype=values_dtype, device=dev)
-    L.call("grws_bcsr_build_fill", nnz, num_rows, num_cols, tile_cols, int(transpose), L.ptr(win), T,
+    return (win,) + _fill(nnz, num_rows, num_cols, tile_cols, transpose, win, T.value, values_dtype, ws, wsb, stream)
+
+
+def _fill(nnz: int, num_rows: int, num_cols: int, tile_cols: int, transpose: bool, win: torch.Tensor, tiles: int,
+          values_dtype: torch.dtype, ws: torch.Tensor, wsb: int, stream) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The fill phase: (column indices, values) of the counted tiles."""
+    out_cols = torch.empty(tiles * tile_cols, dtype=torch.int32, device=win.device)
+    out_vals = torch.empty(tiles * 16 * tile_cols, dtype=values_dtype, device=win.device)
+    L.call("grws_bcsr_build_fill", nnz, num_rows, num_cols, tile_cols, int(transpose), L.ptr(win), tiles,
            L.ptr(out_cols), L.ptr(out_vals), L.dtype_code(values_dtype), L.ptr(ws), wsb, stream)
-    return win, out_cols, out_vals
+    return out_cols, out_vals
 
 
 def csr_to_bcsr_device(num_rows: int, num_cols: int, row_ptr: torch.Tensor, col_idx: torch.Tensor,
@@ -104,14 +109,13 @@ def coo_to_bcsr_device(num_rows: int, num_cols: int, rows: torch.Tensor, cols: t
                   transpose, values_dtype, dev)
 
 
-def bcsr_to_coo(window_offset: torch.Tensor, col_indices: torch.Tensor, values: torch.Tensor,
-                tile_cols: int, num_cols: int):
-    """Edges of a BCSR graph: every slot with a column in [0, num_cols) and a
-    non-zero value.  Returns (rows int32, cols int32, values f32)."""
+def _coo_count(window_offset: torch.Tensor, col_indices: torch.Tensor, values: torch.Tensor, tile_cols: int,
+               num_cols: int, who: str):
+    """(view, edge count, workspace) of grws_bcsr_to_coo_count."""
     dev = window_offset.device
-    L.require_device("bcsr_to_coo", dev, window_offset, col_indices, values)
+    L.require_device(who, dev, window_offset, col_indices, values)
     if not (window_offset.is_contiguous() and col_indices.is_contiguous() and values.is_contiguous()):
-        raise RuntimeError("bcsr_to_coo: the graph arrays must be contiguous")
+        raise RuntimeError(f"{who}: the graph arrays must be contiguous")
     W = window_offset.numel() - 1
     T = col_indices.numel() // tile_cols
     view = L.BcsrView(L.ptr(window_offset), L.ptr(col_indices), L.ptr(values), W, T, 16, tile_cols,
@@ -119,27 +123,41 @@ def bcsr_to_coo(window_offset: torch.Tensor, col_indices: torch.Tensor, values: 
     wsb = int(L.load().grws_bcsr_to_coo_workspace_bytes(T))
     ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
     n = ctypes.c_int64()
-    stream = L.stream_of(dev)
     L.call("grws_bcsr_to_coo_count", ctypes.byref(view), num_cols, L.ptr(ws), wsb, ctypes.byref(n),
-           stream)
-    n = n.value
+           L.stream_of(dev))
+    return view, n.value, ws
+
+
+def bcsr_to_coo(window_offset: torch.Tensor, col_indices: torch.Tensor, values: torch.Tensor,
+                tile_cols: int, num_cols: int):
+    """Edges of a BCSR graph: every slot with a column in [0, num_cols) and a
+    non-zero value.  Returns (rows int32, cols int32, values f32)."""
+    dev = window_offset.device
+    view, n, ws = _coo_count(window_offset, col_indices, values, tile_cols, num_cols, "bcsr_to_coo")
     rows = torch.empty(max(n, 1), dtype=torch.int32, device=dev)
     cols = torch.empty(max(n, 1), dtype=torch.int32, device=dev)
     vals = torch.empty(max(n, 1), dtype=torch.float32, device=dev)
     L.call("grws_bcsr_to_coo_fill", ctypes.byref(view), num_cols, L.ptr(rows), L.ptr(cols),
-           L.ptr(vals), L.ptr(ws), wsb, stream)
+           L.ptr(vals), L.ptr(ws), ws.numel(), L.stream_of(dev))
     return rows[:n], cols[:n], vals[:n]
 
 
 def transpose_arrays(window_offset: torch.Tensor, col_indices: torch.Tensor, values: torch.Tensor,
                      tile_cols: int, num_cols: int, out_tile_cols: Optional[int] = None):
     """BCSR arrays of A^T for a BCSR A with `num_cols` columns.  A^T has
-    ceil(num_cols/16) windows; its columns are A's rows (0 .. 16W-1)."""
-    W = window_offset.numel() - 1
-    rows, cols, vals = bcsr_to_coo(window_offset, col_indices, values, tile_cols, num_cols)
-    return coo_to_bcsr_device(16 * W, num_cols, rows, cols, vals,
-                              tile_cols=out_tile_cols or tile_cols, values_dtype=values.dtype,
-                              transpose=True)
+    ceil(num_cols/16) windows; its columns are A's rows (0 .. 16W-1).  The
+    edges go from the tiles straight to the build's sort keys."""
+    dev = window_offset.device
+    view, nnz, cws = _coo_count(window_offset, col_indices, values, tile_cols, num_cols, "transpose_arrays")
+    rows, tc = 16 * view.num_windows, int(out_tile_cols or tile_cols)
+    win = torch.empty((int(num_cols) + 15) // 16 + 1, dtype=torch.int64, device=dev)
+    wsb = int(L.load().grws_bcsr_build_workspace_bytes(nnz, rows, int(num_cols), 1))
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
+    T = ctypes.c_int64()
+    stream = L.stream_of(dev)
+    L.call("grws_bcsr_transpose_count", ctypes.byref(view), int(num_cols), nnz, L.ptr(cws), cws.numel(), tc,
+           L.ptr(win), L.ptr(ws), wsb, ctypes.byref(T), stream)
+    return (win,) + _fill(nnz, rows, int(num_cols), tc, True, win, T.value, values.dtype, ws, wsb, stream)
 
 
 def transpose(graph):

@@ -125,6 +125,9 @@ _PROTOS = {
                                               ctypes.c_size_t, _c_i64p, _vp]),
     "grws_bcsr_to_coo_fill": (ctypes.c_int, [ctypes.POINTER(BcsrView), ctypes.c_int64, _vp, _vp,
                                              _vp, _vp, ctypes.c_size_t, _vp]),
+    "grws_bcsr_transpose_count": (ctypes.c_int, [ctypes.POINTER(BcsrView), ctypes.c_int64, ctypes.c_int64, _vp,
+                                                 ctypes.c_size_t, ctypes.c_int32, _vp, _vp, ctypes.c_size_t,
+                                                 ctypes.POINTER(ctypes.c_int64), _vp]),
     "grws_coo_to_csr_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64,
                                                           ctypes.c_int64]),
     "grws_coo_to_csr": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64,

@@ -230,6 +230,32 @@ __global__ void keyed_bounds_kernel(const uint64_t* __restrict__ keys, int64_t n
     if (i == n - 1 || (keys[i + 1] & wmask) != w) wend[w] = i + 1;
 }
 
+// The same bounds by two binary searches per window: 54 dependent reads,
+// against a pass over all the keys (0.32 ms for 115M).  Windows without
+// edges keep the zeros they were filled with.
+constexpr int64_t kBoundsSearch = (int64_t)1 << 23;  // keys from which the search is used
+
+__global__ void keyed_bounds_search_kernel(const uint64_t* __restrict__ keys, int64_t n, uint64_t wmask, int64_t W,
+                                           int64_t* __restrict__ wstart, int64_t* __restrict__ wend) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= W) return;
+    int64_t at[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        int64_t lo = 0, hi = n;  // first key of a window >= w + e
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if ((int64_t)(keys[mid] & wmask) < w + e) lo = mid + 1;
+            else hi = mid;
+        }
+        at[e] = lo;
+    }
+    if (at[0] < at[1]) {
+        wstart[w] = at[0];
+        wend[w] = at[1];
+    }
+}
+
 template <typename VT>
 __device__ __forceinline__ void store_value(void* vals, int64_t idx, float v);
 template <>
@@ -1145,6 +1171,24 @@ __device__ __forceinline__ void load_chunk(const void* __restrict__ vals, int64_
     }
 }
 
+// The V columns of chunk slots s0 .. s0 + V - 1 (consecutive slots of one tile
+// row: tc is a multiple of V or V of tc 8), read 16 bytes at a time when
+// ALIGNED (columns 16-byte aligned too).
+template <int V, bool ALIGNED>
+__device__ __forceinline__ void load_cols(const int32_t* __restrict__ cols, int64_t t, int s0, int tc, int32_t* out) {
+    const int32_t* p = cols + t * tc + (s0 & (tc - 1));
+    if constexpr (ALIGNED) {
+#pragma unroll
+        for (int k = 0; k < V; k += 4) {
+            const int4 c = *reinterpret_cast<const int4*>(p + k);
+            out[k] = c.x; out[k + 1] = c.y; out[k + 2] = c.z; out[k + 3] = c.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < V; ++k) out[k] = p[k];
+    }
+}
+
 template <typename VT, bool ALIGNED>
 __global__ __launch_bounds__(256) void tile_nnz_kernel(const int32_t* __restrict__ cols, const void* __restrict__ vals,
                                                        int64_t T, int tc, int64_t num_cols, int32_t* __restrict__ cnt) {
@@ -1158,12 +1202,11 @@ __global__ __launch_bounds__(256) void tile_nnz_kernel(const int32_t* __restrict
             const int64_t t = x / tpb;
             const int s0 = (int)(x % tpb) * V;
             float v[V];
+            int32_t cc[V];
             load_chunk<VT, ALIGNED>(vals, x, v);
+            load_cols<V, ALIGNED>(cols, t, s0, tc, cc);
 #pragma unroll
-            for (int k = 0; k < V; ++k) {
-                const int64_t col = cols[t * tc + (s0 + k) % tc];
-                c += (col >= 0 && col < num_cols && v[k] != 0.0f) ? 1 : 0;
-            }
+            for (int k = 0; k < V; ++k) c += (cc[k] >= 0 && cc[k] < num_cols && v[k] != 0.0f) ? 1 : 0;
         }
         for (int d = tpb / 2; d >= 1; d >>= 1) c += __shfl_xor(c, d, tpb);
         if (x < nch && x % tpb == 0) cnt[x / tpb] = c;
@@ -1182,53 +1225,84 @@ __global__ __launch_bounds__(256) void tile_window_kernel(const int64_t* __restr
     }
 }
 
-template <typename VT, bool ALIGNED>
-__global__ __launch_bounds__(256) void tile_to_coo_kernel(const int32_t* __restrict__ twin,
-                                                          const int32_t* __restrict__ cols,
-                                                          const void* __restrict__ vals, int64_t T, int tc,
-                                                          int64_t num_cols, const int64_t* __restrict__ toff,
-                                                          int32_t* __restrict__ out_rows,
-                                                          int32_t* __restrict__ out_cols,
-                                                          float* __restrict__ out_vals) {
+// Every edge of the tiles: as (row, column, value), or with KEYS as the sort
+// key of the transposed build and its payload.  A wave's 64 chunks are whole
+// consecutive tiles, so its edges take consecutive places from its first
+// tile's toff: they are packed in LDS and written by consecutive lanes (each
+// lane storing its own few edges took 24 store instructions for ~50 edges a
+// wave: 1.85 ms for 114.6M edges in 16x16 f16 tiles).
+template <typename VT, bool ALIGNED, bool KEYS>
+__global__ __launch_bounds__(256) void tile_emit_kernel(const int32_t* __restrict__ twin,
+                                                        const int32_t* __restrict__ cols,
+                                                        const void* __restrict__ vals, int64_t T, int tc,
+                                                        int64_t num_cols, const int64_t* __restrict__ toff,
+                                                        int32_t* __restrict__ out_rows,
+                                                        int32_t* __restrict__ out_cols,
+                                                        float* __restrict__ out_vals, int cbits, int wbits,
+                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ pay) {
     constexpr int V = 16 / (int)sizeof(VT);
+    constexpr int CAP = 64 * V;  // edges of a wave's chunks
+    __shared__ uint64_t srcd[4][CAP];  // row << 32 | column
+    __shared__ float sval[4][CAP];
     const int tpb = 16 * tc / V;
     const int64_t nch = T * tpb;
-    for (int64_t xb = (int64_t)blockIdx.x * 256; xb < nch; xb += (int64_t)gridDim.x * 256) {  // uniform
-        const int64_t x = xb + threadIdx.x;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    for (int64_t xb = (int64_t)blockIdx.x * 256 + wave * kWave; xb < nch; xb += (int64_t)gridDim.x * 256) {
+        const int64_t x = xb + lane;
         const bool in = x < nch;
         const int64_t t = in ? x / tpb : 0;
         const int s0 = in ? (int)(x % tpb) * V : 0;
         float v[V];
         int32_t cc[V];
-        int c = 0;
+        uint32_t ok = 0;
         if (in) {
             load_chunk<VT, ALIGNED>(vals, x, v);
+            load_cols<V, ALIGNED>(cols, t, s0, tc, cc);
 #pragma unroll
-            for (int k = 0; k < V; ++k) {
-                cc[k] = cols[t * tc + (s0 + k) % tc];
-                c += (cc[k] >= 0 && cc[k] < num_cols && v[k] != 0.0f) ? 1 : 0;
-            }
+            for (int k = 0; k < V; ++k)
+                ok |= (cc[k] >= 0 && cc[k] < num_cols && v[k] != 0.0f) ? 1u << k : 0u;
         }
-        // exclusive prefix over the tile's chunks (consecutive lanes)
+        const int c = __popc(ok);
         int inc = c;
-        const int gl = (int)(threadIdx.x % tpb);
-        for (int d = 1; d < tpb; d <<= 1) {
-            const int y = __shfl_up(inc, d, tpb);
-            if (gl >= d) inc += y;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int y = __shfl_up(inc, d, kWave);
+            if (lane >= d) inc += y;
         }
-        if (in && c) {
-            int64_t pos = toff[t] + inc - c;
-            const int64_t row0 = 16 * (int64_t)twin[t];
+        const int total = __shfl(inc, kWave - 1, kWave);
+        if (c) {
+            int at = inc - c;
+            const uint64_t row = (uint64_t)(16 * (int64_t)twin[t] + s0 / tc);
 #pragma unroll
             for (int k = 0; k < V; ++k) {
-                if (cc[k] >= 0 && cc[k] < num_cols && v[k] != 0.0f) {
-                    out_rows[pos] = (int32_t)(row0 + (s0 + k) / tc);
-                    out_cols[pos] = cc[k];
-                    out_vals[pos] = v[k];
-                    ++pos;
+                if (ok >> k & 1u) {
+                    srcd[wave][at] = (row << 32) | (uint32_t)cc[k];
+                    sval[wave][at] = v[k];
+                    ++at;
                 }
             }
         }
+        // the wave reads what its own lanes wrote (LDS operations of a wave
+        // run in order; the fences keep the compiler from reordering them)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int64_t base = toff[xb / tpb];
+        for (int i = lane; i < total; i += kWave) {
+            const uint64_t rc = srcd[wave][i];
+            const int64_t r = (int64_t)(rc >> 32), cl = (int64_t)(uint32_t)rc;
+            if constexpr (KEYS) {
+                keys[base + i] = edge_key(cl, r, cbits, wbits);
+                pay[base + i] = __float_as_uint(sval[wave][i]);
+            } else {
+                out_rows[base + i] = (int32_t)r;
+                out_cols[base + i] = (int32_t)cl;
+                out_vals[base + i] = sval[wave][i];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 }
 
@@ -1323,28 +1397,13 @@ extern "C" size_t grws_bcsr_build_workspace_bytes(int64_t nnz, int64_t num_rows,
     return nc.s.used + 256;
 }
 
-extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows, const int32_t* cols,
-                                     const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols,
-                                     int32_t tile_cols, int32_t transpose, int64_t* window_offset, void* workspace,
-                                     size_t workspace_bytes, int64_t* num_tiles_out, void* stream_) {
-    clear_error();
-    hipStream_t stream = as_stream(stream_);
-    GRWS_TRY(refuse_capture(stream, "bcsr_build_count"));
-    GRWS_CHECK_ARG(nnz >= 0 && num_rows >= 0 && num_cols >= 0, "bcsr_build: negative size");
-    GRWS_CHECK_ARG(num_rows <= INT32_MAX && num_cols <= INT32_MAX, "bcsr_build: dimensions exceed int32 ids");
-    GRWS_CHECK_ARG(nnz <= (int64_t)UINT32_MAX, "bcsr_build: more than 2^32-1 edges");
-    GRWS_CHECK_ARG(tile_cols == 8 || tile_cols == 16, "bcsr_build: tile_cols must be 8 or 16 (got %d)", tile_cols);
-    GRWS_CHECK_ARG(window_offset && num_tiles_out, "bcsr_build: null output");
-    GRWS_CHECK_ARG(row_ptr == nullptr || rows == nullptr, "bcsr_build: pass only one of row_ptr and rows");
-    if (nnz > 0) GRWS_CHECK_ARG(row_ptr != nullptr || rows != nullptr, "bcsr_build: pass row_ptr or rows");
-    if (nnz > 0) GRWS_CHECK_ARG(cols != nullptr, "bcsr_build: null cols");
-    if (row_ptr) GRWS_CHECK_ARG(num_rows > 0 || nnz == 0, "bcsr_build: edges without rows");
-    BuildShape s = build_shape(nnz, num_rows, num_cols, transpose);
-    Carver cv(workspace, workspace_bytes);
-    BuildWs w;
-    carve_build(cv, s, &w);
-    if (!cv.ok) return set_error(GRWS_E_CAPACITY, "bcsr_build: workspace too small (%zu < %zu)", workspace_bytes, cv.used);
-
+// The count phase after its checks.  emit_keys(wbits) writes the nnz edge
+// keys of that layout (edge_key) and their values to w.ka / w.va.
+template <typename EmitKeys>
+static int build_count(const BuildShape& s, BuildWs& w, const int64_t* row_ptr, const int32_t* cols,
+                       const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols, int32_t tile_cols,
+                       int32_t transpose, int64_t* window_offset, int64_t* num_tiles_out, hipStream_t stream,
+                       EmitKeys emit_keys) {
     GRWS_TRY(fill_i32(w.err, 4, 0, stream));  // error flags, big windows, path of the fill, huge windows
     if (s.W == 0) {
         GRWS_TRY(fill_i64(window_offset, 1, 0, stream));
@@ -1379,19 +1438,14 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
         per_window = (h[0] & kErrRowPtr) == 0 && h[3] == 0;
         nbig = h[1];
     } else if (nnz > 0 && s.C <= ((int64_t)1 << 27)) {
-        if (rows) {
-            hipLaunchKernelGGL(build_keys_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, row_ptr, rows, cols,
-                               values, nnz, num_rows, num_cols, (int)transpose, s.cbits, kwbits, w.ka, w.va, w.err);
-        } else {
-            const int64_t wg = std::min<int64_t>((num_rows + 3) / 4, 65536);
-            hipLaunchKernelGGL(build_keys_rows_kernel, dim3((unsigned)std::max<int64_t>(wg, 1)), dim3(256), 0, stream,
-                               row_ptr, cols, values, nnz, num_rows, num_cols, (int)transpose, s.cbits, kwbits, w.ka,
-                               w.va, w.err);
-        }
-        GRWS_LAUNCH_CHECK();
+        GRWS_TRY(emit_keys(kwbits));
         GRWS_TRY(radix_sort_pairs(w.ka, w.va, w.kb, w.vb, nnz, kwbits, w.sort_ws, w.sort_bytes, stream, &kalt));
-        hipLaunchKernelGGL(keyed_bounds_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, kalt ? w.kb : w.ka, nnz,
-                           ((uint64_t)1 << kwbits) - 1, w.wstart, w.wend);
+        if (nnz >= kBoundsSearch)
+            hipLaunchKernelGGL(keyed_bounds_search_kernel, dim3(grid_for(s.W, 64)), dim3(64), 0, stream,
+                               kalt ? w.kb : w.ka, nnz, ((uint64_t)1 << kwbits) - 1, s.W, w.wstart, w.wend);
+        else
+            hipLaunchKernelGGL(keyed_bounds_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, kalt ? w.kb : w.ka, nnz,
+                               ((uint64_t)1 << kwbits) - 1, w.wstart, w.wend);
         GRWS_LAUNCH_CHECK();
         hipLaunchKernelGGL(keyed_big_kernel, dim3(grid_for(s.W)), dim3(kBlk), 0, stream, w.wstart, w.wend, s.W,
                            w.blist, w.err);
@@ -1473,18 +1527,7 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
     }
     bool alt = false;
     if (nnz > 0 && !per_window) {
-        if (rows) {
-            hipLaunchKernelGGL(build_keys_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, row_ptr, rows, cols,
-                               values, nnz, num_rows, num_cols, (int)transpose, s.cbits, 0, w.ka, w.va, w.err);
-        } else {
-            // every edge lies in some row's range (check_row_ptr_kernel flags
-            // a row pointer that does not cover [0, nnz) exactly)
-            const int64_t wg = std::min<int64_t>((num_rows + 3) / 4, 65536);
-            hipLaunchKernelGGL(build_keys_rows_kernel, dim3((unsigned)std::max<int64_t>(wg, 1)), dim3(256), 0, stream,
-                               row_ptr, cols, values, nnz, num_rows, num_cols, (int)transpose, s.cbits, 0, w.ka,
-                               w.va, w.err);
-        }
-        GRWS_LAUNCH_CHECK();
+        GRWS_TRY(emit_keys(0));
         GRWS_TRY(radix_sort_pairs(w.ka, w.va, w.kb, w.vb, nnz, s.bits, w.sort_ws, w.sort_bytes, stream, &alt));
         const uint64_t* k = alt ? w.kb : w.ka;
         hipLaunchKernelGGL(unique_flag_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, k, nnz, w.uflag);
@@ -1508,6 +1551,46 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
     GRWS_TRY(report_input_error(e, "bcsr_build"));
     *num_tiles_out = T;
     return GRWS_OK;
+}
+
+extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows, const int32_t* cols,
+                                     const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols,
+                                     int32_t tile_cols, int32_t transpose, int64_t* window_offset, void* workspace,
+                                     size_t workspace_bytes, int64_t* num_tiles_out, void* stream_) {
+    clear_error();
+    hipStream_t stream = as_stream(stream_);
+    GRWS_TRY(refuse_capture(stream, "bcsr_build_count"));
+    GRWS_CHECK_ARG(nnz >= 0 && num_rows >= 0 && num_cols >= 0, "bcsr_build: negative size");
+    GRWS_CHECK_ARG(num_rows <= INT32_MAX && num_cols <= INT32_MAX, "bcsr_build: dimensions exceed int32 ids");
+    GRWS_CHECK_ARG(nnz <= (int64_t)UINT32_MAX, "bcsr_build: more than 2^32-1 edges");
+    GRWS_CHECK_ARG(tile_cols == 8 || tile_cols == 16, "bcsr_build: tile_cols must be 8 or 16 (got %d)", tile_cols);
+    GRWS_CHECK_ARG(window_offset && num_tiles_out, "bcsr_build: null output");
+    GRWS_CHECK_ARG(row_ptr == nullptr || rows == nullptr, "bcsr_build: pass only one of row_ptr and rows");
+    if (nnz > 0) GRWS_CHECK_ARG(row_ptr != nullptr || rows != nullptr, "bcsr_build: pass row_ptr or rows");
+    if (nnz > 0) GRWS_CHECK_ARG(cols != nullptr, "bcsr_build: null cols");
+    if (row_ptr) GRWS_CHECK_ARG(num_rows > 0 || nnz == 0, "bcsr_build: edges without rows");
+    BuildShape s = build_shape(nnz, num_rows, num_cols, transpose);
+    Carver cv(workspace, workspace_bytes);
+    BuildWs w;
+    carve_build(cv, s, &w);
+    if (!cv.ok) return set_error(GRWS_E_CAPACITY, "bcsr_build: workspace too small (%zu < %zu)", workspace_bytes, cv.used);
+
+    return build_count(s, w, row_ptr, cols, values, nnz, num_rows, num_cols, tile_cols, transpose, window_offset,
+                       num_tiles_out, stream, [&](int wbits) -> int {
+        if (rows) {
+            hipLaunchKernelGGL(build_keys_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, row_ptr, rows, cols,
+                               values, nnz, num_rows, num_cols, (int)transpose, s.cbits, wbits, w.ka, w.va, w.err);
+        } else {
+            // every edge lies in some row's range (check_row_ptr_kernel flags
+            // a row pointer that does not cover [0, nnz) exactly)
+            const int64_t wg = std::min<int64_t>((num_rows + 3) / 4, 65536);
+            hipLaunchKernelGGL(build_keys_rows_kernel, dim3((unsigned)std::max<int64_t>(wg, 1)), dim3(256), 0, stream,
+                               row_ptr, cols, values, nnz, num_rows, num_cols, (int)transpose, s.cbits, wbits, w.ka,
+                               w.va, w.err);
+        }
+        GRWS_LAUNCH_CHECK();
+        return GRWS_OK;
+    });
 }
 
 extern "C" int grws_bcsr_build_fill(int64_t nnz, int64_t num_rows, int64_t num_cols, int32_t tile_cols,
@@ -1619,6 +1702,45 @@ static int check_bcsr(const grws_bcsr* A, const char* who) {
     return GRWS_OK;
 }
 
+// Values and columns that the 16-byte reads may take.
+static bool tiles_aligned(const grws_bcsr* A) {
+    return ((reinterpret_cast<uintptr_t>(A->values) | reinterpret_cast<uintptr_t>(A->col_indices)) & 15) == 0;
+}
+
+static int launch_tile_windows(const grws_bcsr* A, int32_t* twin, hipStream_t stream) {
+    GRWS_TRY(fill_i32(twin, A->num_tiles, 0, stream));
+    hipLaunchKernelGGL(tile_window_kernel, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(A->num_windows, 8192))),
+                       dim3(256), 0, stream, A->window_offset, A->num_windows, A->num_tiles, twin);
+    GRWS_LAUNCH_CHECK();
+    return GRWS_OK;
+}
+
+template <bool KEYS>
+static int launch_tile_emit(const grws_bcsr* A, int64_t num_cols, const int32_t* twin, const int64_t* toff,
+                            int32_t* rows, int32_t* cols, float* values, int cbits, int wbits, uint64_t* keys,
+                            uint32_t* pay, hipStream_t stream) {
+    const int64_t nch = A->num_tiles * 16 * A->tile_cols / (16 / dtype_size(A->values_dtype));
+    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((nch + 255) / 256, 65536));
+    const bool al = tiles_aligned(A);
+#define GRWS_TILE_EMIT(VT)                                                                                         \
+    if (al)                                                                                                        \
+        hipLaunchKernelGGL((tile_emit_kernel<VT, true, KEYS>), dim3(grid), dim3(256), 0, stream, twin,             \
+                           A->col_indices, A->values, A->num_tiles, A->tile_cols, num_cols, toff, rows, cols,      \
+                           values, cbits, wbits, keys, pay);                                                       \
+    else                                                                                                           \
+        hipLaunchKernelGGL((tile_emit_kernel<VT, false, KEYS>), dim3(grid), dim3(256), 0, stream, twin,            \
+                           A->col_indices, A->values, A->num_tiles, A->tile_cols, num_cols, toff, rows, cols,      \
+                           values, cbits, wbits, keys, pay)
+    switch (A->values_dtype) {
+        case GRWS_F32: GRWS_TILE_EMIT(float); break;
+        case GRWS_F16: GRWS_TILE_EMIT(_Float16); break;
+        default: GRWS_TILE_EMIT(__hip_bfloat16); break;
+    }
+#undef GRWS_TILE_EMIT
+    GRWS_LAUNCH_CHECK();
+    return GRWS_OK;
+}
+
 extern "C" int grws_bcsr_to_coo_count(const grws_bcsr* A, int64_t num_cols, void* workspace, size_t workspace_bytes,
                                       int64_t* nnz_out, void* stream_) {
     clear_error();
@@ -1637,7 +1759,7 @@ extern "C" int grws_bcsr_to_coo_count(const grws_bcsr* A, int64_t num_cols, void
     GRWS_TRY(coo_ws(workspace, workspace_bytes, T, &cnt, &toff, &sws, &sb));
     const int64_t nch = T * 16 * A->tile_cols / (16 / dtype_size(A->values_dtype));
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((nch + 255) / 256, 65536));
-    const bool al = (reinterpret_cast<uintptr_t>(A->values) & 15) == 0;
+    const bool al = tiles_aligned(A);
 #define GRWS_TILE_NNZ(VT)                                                                                          \
     if (al)                                                                                                        \
         hipLaunchKernelGGL((tile_nnz_kernel<VT, true>), dim3(grid), dim3(256), 0, stream, A->col_indices,          \
@@ -1676,27 +1798,8 @@ extern "C" int grws_bcsr_to_coo_fill(const grws_bcsr* A, int64_t num_cols, int32
     GRWS_TRY(coo_ws(workspace, workspace_bytes, T, &cnt, &toff, &sws, &sb));
     // the count's per-tile counts are spent (toff holds their scan): the
     // array takes each tile's window
-    GRWS_TRY(fill_i32(cnt, T, 0, stream));
-    hipLaunchKernelGGL(tile_window_kernel, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(A->num_windows, 8192))),
-                       dim3(256), 0, stream, A->window_offset, A->num_windows, T, cnt);
-    GRWS_LAUNCH_CHECK();
-    const int64_t nch = T * 16 * A->tile_cols / (16 / dtype_size(A->values_dtype));
-    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((nch + 255) / 256, 65536));
-    const bool al = (reinterpret_cast<uintptr_t>(A->values) & 15) == 0;
-#define GRWS_TILE_COO(VT)                                                                                          \
-    if (al)                                                                                                        \
-        hipLaunchKernelGGL((tile_to_coo_kernel<VT, true>), dim3(grid), dim3(256), 0, stream, cnt, A->col_indices,  \
-                           A->values, T, A->tile_cols, num_cols, toff, rows, cols, values);                        \
-    else                                                                                                           \
-        hipLaunchKernelGGL((tile_to_coo_kernel<VT, false>), dim3(grid), dim3(256), 0, stream, cnt, A->col_indices, \
-                           A->values, T, A->tile_cols, num_cols, toff, rows, cols, values)
-    switch (A->values_dtype) {
-        case GRWS_F32: GRWS_TILE_COO(float); break;
-        case GRWS_F16: GRWS_TILE_COO(_Float16); break;
-        default: GRWS_TILE_COO(__hip_bfloat16); break;
-    }
-#undef GRWS_TILE_COO
-    GRWS_LAUNCH_CHECK();
+    GRWS_TRY(launch_tile_windows(A, cnt, stream));
+    GRWS_TRY(launch_tile_emit<false>(A, num_cols, cnt, toff, rows, cols, values, 0, 0, nullptr, nullptr, stream));
     return GRWS_OK;
 }
 
@@ -1760,4 +1863,41 @@ extern "C" int grws_coo_to_csr(const int32_t* src, const int32_t* dst, const flo
     GRWS_TRY(read_error_flag(err, stream, &e));
     GRWS_HIP(hipStreamSynchronize(stream));
     return report_input_error(e, "coo_to_csr");
+}
+
+extern "C" int grws_bcsr_transpose_count(const grws_bcsr* A, int64_t num_cols, int64_t nnz, void* coo_workspace,
+                                         size_t coo_workspace_bytes, int32_t tile_cols, int64_t* window_offset,
+                                         void* workspace, size_t workspace_bytes, int64_t* num_tiles_out,
+                                         void* stream_) {
+    clear_error();
+    hipStream_t stream = as_stream(stream_);
+    GRWS_TRY(refuse_capture(stream, "bcsr_transpose_count"));
+    GRWS_TRY(check_bcsr(A, "bcsr_transpose"));
+    GRWS_CHECK_ARG(nnz >= 0 && num_cols >= 0, "bcsr_transpose: negative size");
+    GRWS_CHECK_ARG(num_cols <= INT32_MAX, "bcsr_transpose: num_cols exceeds int32 column ids");
+    GRWS_CHECK_ARG(nnz <= (int64_t)UINT32_MAX && nnz <= A->num_tiles * 16 * A->tile_cols,
+                   "bcsr_transpose: nnz is not the count of the graph's edges");
+    GRWS_CHECK_ARG(tile_cols == 8 || tile_cols == 16, "bcsr_transpose: tile_cols must be 8 or 16 (got %d)", tile_cols);
+    GRWS_CHECK_ARG(window_offset && num_tiles_out, "bcsr_transpose: null output");
+    const int64_t rows = 16 * A->num_windows;
+    const BuildShape s = build_shape(nnz, rows, num_cols, 1);
+    Carver cv(workspace, workspace_bytes);
+    BuildWs w;
+    carve_build(cv, s, &w);
+    if (!cv.ok)
+        return set_error(GRWS_E_CAPACITY, "bcsr_transpose: workspace too small (%zu < %zu)", workspace_bytes, cv.used);
+    int32_t* twin = nullptr;
+    int64_t* toff = nullptr;
+    if (nnz > 0) {
+        char* sws;
+        size_t sb;
+        GRWS_TRY(coo_ws(coo_workspace, coo_workspace_bytes, A->num_tiles, &twin, &toff, &sws, &sb));
+        // the per-tile counts are spent (toff holds their scan)
+        GRWS_TRY(launch_tile_windows(A, twin, stream));
+    }
+    return build_count(s, w, nullptr, nullptr, nullptr, nnz, rows, num_cols, tile_cols, 1, window_offset,
+                       num_tiles_out, stream, [&](int wbits) -> int {
+        return launch_tile_emit<true>(A, num_cols, twin, toff, nullptr, nullptr, nullptr, s.cbits, wbits, w.ka, w.va,
+                                      stream);
+    });
 }

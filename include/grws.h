@@ -360,6 +360,16 @@ int grws_bcsr_to_coo_count(const grws_bcsr* A, int64_t num_cols, void* workspace
 int grws_bcsr_to_coo_fill(const grws_bcsr* A, int64_t num_cols, int32_t* rows, int32_t* cols,
                           float* values, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Count phase of the transpose's build from the BCSR itself: after
+ * grws_bcsr_to_coo_count (its nnz and its workspace, kept as it left it),
+ * the edges go to the sort without the COO arrays between.  Same result and
+ * workspace as grws_bcsr_build_count(rows, cols, values of the COO, nnz,
+ * 16 * num_windows, num_cols, transpose = 1); grws_bcsr_build_fill follows. */
+int grws_bcsr_transpose_count(const grws_bcsr* A, int64_t num_cols, int64_t nnz, void* coo_workspace,
+                              size_t coo_workspace_bytes, int32_t tile_cols, int64_t* window_offset,
+                              void* workspace, size_t workspace_bytes, int64_t* num_tiles_out,
+                              void* stream);
+
 /* COO -> CSR, replacing BCSRGraph._coo_to_csr (data/bcsr.py:162-187):
  * stable sort by (src, dst) (the reference sorts on src*num_rows+dst with a
  * non-stable argsort, :170-171), row_ptr int64 [num_rows+1], col_idx = dst,

@@ -94,11 +94,8 @@ class BCSRGraph:
         num_nodes = g.num_nodes()
         src, dst = g.edges()
         edge_weights = g.edata.get("weight", None)
-        num_edges, row_ptr, col_idx, values = cls._coo_to_csr(num_nodes, src, dst, edge_weights,
-                                                              device, num_cols=num_nodes)
-        return cls._from_csr(num_rows=num_nodes, row_ptr=row_ptr, col_idx=col_idx,
-                             edge_values=values, tile_rows=tile_rows, tile_cols=tile_cols,
-                             device=device, num_cols=num_nodes, values_dtype=values_dtype)
+        return cls._from_coo(num_nodes, num_nodes, src, dst, edge_weights, device, tile_rows, tile_cols,
+                             values_dtype)
 
     @classmethod
     def from_mtx(cls, filepath: str, index_base: int = 0, undirected: bool = False,
@@ -191,6 +188,30 @@ class BCSRGraph:
         return num_edges, row_ptr, col_idx, values
 
     @classmethod
+    def _from_coo(cls, num_rows: int, num_cols: int, rows: torch.Tensor, cols: torch.Tensor,
+                  edge_weights: Optional[torch.Tensor], device: torch.device, tile_rows: int, tile_cols: int,
+                  values_dtype: Optional[torch.dtype]) -> "BCSRGraph":
+        """COO -> BCSR.  Edges on the graph's own device are built without
+        the CSR between: the build sorts them by window only (two 8-bit
+        passes on 14,561 windows, against five by (row, column)), and of
+        duplicate edges the last in input order wins either way."""
+        from .. import builder
+        dev = torch.device(device)
+        here = rows.is_cuda and dev.type == "cuda" and rows.device.index == (
+            torch.cuda.current_device() if dev.index is None else dev.index)
+        if here and tile_rows == 16 and builder.available():
+            win, bcols, vals = builder.coo_to_bcsr_device(int(num_rows), int(num_cols), rows, cols, edge_weights,
+                                                          tile_cols=tile_cols,
+                                                          values_dtype=values_dtype or torch.float32)
+            return cls(num_nodes=int(num_rows), num_edges=int(rows.numel()), tile_rows=tile_rows,
+                       tile_cols=tile_cols, window_offset=win, original_col_indices=bcols, values_condensed=vals,
+                       device=device, num_rows=int(num_rows), num_cols=int(num_cols), values_dtype=values_dtype)
+        _, row_ptr, col_idx, values = cls._coo_to_csr(num_rows, rows, cols, edge_weights, device, num_cols=num_cols)
+        return cls._from_csr(num_rows=num_rows, row_ptr=row_ptr, col_idx=col_idx, edge_values=values,
+                             tile_rows=tile_rows, tile_cols=tile_cols, device=device, num_cols=num_cols,
+                             values_dtype=values_dtype)
+
+    @classmethod
     def _from_csr(cls, num_rows: int, row_ptr: torch.Tensor, col_idx: torch.Tensor,
                   edge_values: torch.Tensor, tile_rows: int, tile_cols: int, device: torch.device,
                   num_cols: Optional[int] = None,
@@ -252,11 +273,7 @@ class BCSRGraph:
         num_cols = block.num_src_nodes()
         src, dst = block.edges()
         edge_weights = block.edata.get("weight", None) if "weight" in block.edata else None
-        num_edges, row_ptr, col_idx, values = cls._coo_to_csr(num_rows, dst, src, edge_weights,
-                                                              device, num_cols=num_cols)
-        return cls._from_csr(num_rows=num_rows, row_ptr=row_ptr, col_idx=col_idx,
-                             edge_values=values, tile_rows=tile_rows, tile_cols=tile_cols,
-                             device=device, num_cols=num_cols, values_dtype=values_dtype)
+        return cls._from_coo(num_rows, num_cols, dst, src, edge_weights, device, tile_rows, tile_cols, values_dtype)
 
     # ---------------- MI355X additions ----------------
     def spmm_plan(self, n_cols: int):

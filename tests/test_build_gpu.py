@@ -11,6 +11,7 @@ import torch
 import oracle
 from graph_rws_amd import builder, core, synth
 from graph_rws_amd.core._lib import GrwsError
+from graph_rws_amd.data import BCSRGraph
 
 pytestmark = pytest.mark.gpu
 
@@ -599,3 +600,80 @@ def test_large_sort_tiles_are_stable(cuda_device, n, spread):
     perm = torch.sort(src.long() * 300 + dst.long(), stable=True).indices
     assert torch.equal(ci, dst[perm]) and torch.equal(va, w[perm])
     assert torch.equal(rp[1:] - rp[:-1], torch.bincount(src.long(), minlength=rows))
+
+
+@pytest.mark.parametrize("vdt,tc,offset", [(torch.float32, 8, 0), (torch.float32, 16, 1), (torch.float16, 16, 0),
+                                           (torch.float16, 8, 3), (torch.bfloat16, 16, 0)])
+def test_transpose_keys_from_tiles_equal_the_coo_route(cuda_device, vdt, tc, offset):
+    """The transpose built from the tiles' own keys against the COO arrays
+    built as before, on ragged windows, dropped columns, explicit zeros,
+    empty windows and misaligned values."""
+    print(f"case transpose keys {vdt} tc={tc} offset={offset}", flush=True)
+    g = synth.chung_lu(1003, 30000, 2.1, seed=4)
+    hw, hc, hv = _host(g, tc)
+    hv = hv.to(vdt)
+    hv.view(-1)[::5] = 0
+    buf = torch.empty(hv.numel() + offset, dtype=vdt, device=cuda_device)
+    dv = buf[offset:]
+    dv.copy_(hv.view(-1).to(cuda_device))
+    w, c = hw.to(cuda_device), hc.to(cuda_device)
+    for ncols in (g.num_nodes, g.num_nodes - 37, 1):
+        got = builder.transpose_arrays(w, c, dv, tc, ncols)
+        r, cc, v = builder.bcsr_to_coo(w, c, dv, tc, ncols)
+        ref = builder.coo_to_bcsr_device(16 * (w.numel() - 1), ncols, r, cc, v, tile_cols=tc, values_dtype=vdt,
+                                         transpose=True)
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b)
+    empty = builder.transpose_arrays(torch.zeros(4, dtype=torch.int64, device=cuda_device), c[:0], dv[:0], tc, 20)
+    assert empty[0].tolist() == [0, 0, 0] and empty[1].numel() == 0 and empty[2].numel() == 0
+
+
+class _Loaded:
+    """What a graph loader hands over (num_nodes, edges, edata, device), also
+    as a message-flow block."""
+
+    def __init__(self, rows, cols, src, dst, w, device):
+        self.rows, self.cols, self.src, self.dst, self.device = rows, cols, src, dst, device
+        self.edata = {} if w is None else {"weight": w}
+
+    def num_nodes(self):
+        return self.rows
+
+    def num_dst_nodes(self):
+        return self.rows
+
+    def num_src_nodes(self):
+        return self.cols
+
+    def edges(self):
+        return self.src, self.dst
+
+
+@pytest.mark.parametrize("tc,vdt", [(8, torch.float32), (16, torch.float16), (16, torch.bfloat16)])
+@pytest.mark.parametrize("n,m,nnz", [(1, 1, 0), (33, 33, 0), (17, 17, 40), (300, 300, 9000), (5000, 40, 60000)])
+def test_loaded_edges_equal_the_csr_route(cuda_device, tc, vdt, n, m, nnz):
+    """from_dgl / from_dgl_block of device edges (built without the CSR)
+    against the same edges sorted to a CSR first: any order, duplicates, int32
+    and int64 ids, strided ids, with and without weights."""
+    print(f"case loaded edges n={n} m={m} nnz={nnz} tc={tc} {vdt}", flush=True)
+    g = torch.Generator().manual_seed(n + m + nnz)
+    r = torch.randint(0, n, (nnz,), generator=g)
+    c = torch.randint(0, m, (nnz,), generator=g)
+    f = torch.randn(nnz, generator=g)
+    for ids, weights in ((torch.int64, f), (torch.int32, None), (torch.int64, f.double())):
+        for strided in (False, True):
+            def dev(t):
+                t = t.to(cuda_device)
+                return torch.stack([t, t], 1)[:, 0] if strided else t
+            hr, hc = dev(r.to(ids)), dev(c.to(ids))
+            w = None if weights is None else weights.to(cuda_device)
+            _, rp, ci, va = BCSRGraph._coo_to_csr(n, hr, hc, w, cuda_device, num_cols=m)
+            ref = BCSRGraph._from_csr(n, rp, ci, va, 16, tc, cuda_device, num_cols=m, values_dtype=vdt)
+            made = [BCSRGraph.from_dgl_block(_Loaded(n, m, hc, hr, w, cuda_device), tile_cols=tc, values_dtype=vdt)]
+            if n == m:
+                made.append(BCSRGraph.from_dgl(_Loaded(n, m, hr, hc, w, torch.device("cuda")), tile_cols=tc,
+                                               values_dtype=vdt))
+            for got in made:
+                for a in ("window_offset", "original_col_indices", "values_condensed"):
+                    assert torch.equal(getattr(ref, a), getattr(got, a)), a
+                assert (ref.num_edges, ref.num_rows, ref.num_cols) == (got.num_edges, got.num_rows, got.num_cols)

@@ -131,6 +131,19 @@ struct SideStream {
     SideStream(const SideStream&) = delete;
     SideStream& operator=(const SideStream&) = delete;
     int fork() { return side_fork(main, &side); }
+    // the side stream waits for what the main stream holds by now (a first
+    // fork when there is none; a forked stream stays forked, so an error here
+    // still joins the work it already has)
+    int fork_again() {
+        if (side == main) return fork();
+        hipEvent_t ev;
+        GRWS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        hipError_t e = hipEventRecord(ev, main);
+        if (e == hipSuccess) e = hipStreamWaitEvent(side, ev, 0);
+        (void)hipEventDestroy(ev);
+        GRWS_HIP(e);
+        return GRWS_OK;
+    }
     // fork onto a caller-owned stream `s` instead (a capture's own second
     // stream: under capture the event wait joins `s` into the capture, and
     // no other caller shares it); null keeps the work on `main`

@@ -1170,12 +1170,15 @@ HopCaps hop_caps(int64_t num_seeds, const int32_t* fanouts, int H, int tc, int64
 
 struct BatchWs {
     int64_t* edge_src;
-    float* edge_val;
-    int32_t* src_local;
+    // a transposed hop's slots are its own (its transpose is built while the
+    // next hops sample); the other hops share theirs
+    float* edge_val[kMaxHops];
+    int32_t* src_local[kMaxHops];
     int32_t* grpoff;
     int32_t* slicesum;
     int32_t* sliceoff;
     int32_t* wtiles;
+    int32_t* twtiles;
     int64_t* out;
     char* scan_ws;
     size_t scan_bytes;
@@ -1189,8 +1192,9 @@ struct BatchWs {
 
 template <typename C>
 void carve_batch(C& cv, const HopCaps& c, int H, int64_t num_nodes, const int32_t* thops, BatchWs* w) {
-    int64_t emax = 1, wmax = 1, etmax = 0;
+    int64_t emax = 1, wmax = 1, etmax = 0, eshared = 1;
     for (int h = 0; h < H; ++h) {
+        if (!(thops && thops[h])) eshared = c.E[h] > eshared ? c.E[h] : eshared;
         emax = c.E[h] > emax ? c.E[h] : emax;
         wmax = c.W[h] > wmax ? c.W[h] : wmax;
         if (thops && thops[h]) {
@@ -1199,12 +1203,18 @@ void carve_batch(C& cv, const HopCaps& c, int H, int64_t num_nodes, const int32_
         }
     }
     w->edge_src = cv.template take<int64_t>(emax);
-    w->edge_val = cv.template take<float>(emax);
-    w->src_local = cv.template take<int32_t>(emax);
+    float* ev = cv.template take<float>(eshared);
+    int32_t* sl = cv.template take<int32_t>(eshared);
+    for (int h = 0; h < kMaxHops; ++h) {
+        const bool own = h < H && thops && thops[h];
+        w->edge_val[h] = own ? cv.template take<float>(c.E[h]) : ev;
+        w->src_local[h] = own ? cv.template take<int32_t>(c.E[h]) : sl;
+    }
     w->grpoff = cv.template take<int32_t>(group_count(num_nodes) + 1);
     w->slicesum = cv.template take<int32_t>(group_count(num_nodes) / kSliceGroups + 2);
     w->sliceoff = cv.template take<int32_t>(group_count(num_nodes) / kSliceGroups + 2);
     w->wtiles = cv.template take<int32_t>(wmax + 1);
+    w->twtiles = etmax > 0 ? cv.template take<int32_t>(wmax + 1) : nullptr;
     w->out = cv.template take<int64_t>(5 * kMaxHops + 4);
     w->scan_bytes = scan_workspace_bytes(wmax);
     w->scan_ws = cv.template take<char>(w->scan_bytes);
@@ -1664,9 +1674,15 @@ static int sample_blocks_impl(const int64_t* indptr, const int32_t* indices, int
         hipLaunchKernelGGL(mh_start_kernel, dim3(1), dim3(64), 0, stream, num_seeds_dev, num_seeds, ctr);
         GRWS_LAUNCH_CHECK();
     }
+    // A hop's transpose is a chain of ~10 small dependent kernels (45 us of a
+    // 1,024-seed batch's 258 us); on the device's second stream it runs beside
+    // the next hops' sampling.  Without a next hop it stays on the caller's.
+    SideStream ss(stream);
     for (int h = 0; h < H; ++h) {
         const int k = fanouts[h];
         const int64_t Fc = c.F[h], Wc = c.W[h];
+        float* edge_val = w.edge_val[h];
+        int32_t* src_local = w.src_local[h];
         const int64_t* fr = h == 0 ? seeds : next_frontier[h - 1];
         if (h == 0) {
             hipLaunchKernelGGL(mh_seed_kernel, dim3(grid_for(Fc)), dim3(kBlk), 0, stream, indptr, nnz, num_nodes,
@@ -1675,19 +1691,19 @@ static int sample_blocks_impl(const int64_t* indptr, const int32_t* indices, int
         }
         hipLaunchKernelGGL(mh_sample_kernel, dim3(grid_for(Fc, kWavesPerBlock)), dim3(kBlk), 0, stream, indptr,
                            indices, nnz, num_nodes, fr, F0, h, k, seed, node_map, bitmap, grpcnt, w.edge_src,
-                           w.edge_val, ctr);
+                           edge_val, ctr);
         GRWS_LAUNCH_CHECK();
         const int64_t nslices = (l.groups + kSliceGroups - 1) / kSliceGroups;
         hipLaunchKernelGGL(mh_group_scan_kernel, dim3((unsigned)nslices), dim3(kBlk), 0, stream, grpcnt, l.groups,
                            w.grpoff, w.slicesum, w.sliceoff, nslices, F0, h, ctr);
         GRWS_LAUNCH_CHECK();
         hipLaunchKernelGGL(mh_wcount_kernel, dim3((unsigned)Wc), dim3(kBlk), 0, stream, fr, F0, h, k, num_nodes,
-                           w.edge_src, node_map, (int)(h + 1 < H), bitmap, w.grpoff, w.sliceoff, w.src_local,
+                           w.edge_src, node_map, (int)(h + 1 < H), bitmap, w.grpoff, w.sliceoff, src_local,
                            next_frontier[h], tc, w.wtiles, ctr);
         GRWS_LAUNCH_CHECK();
 #define GRWS_MH_WINDOWS(VT)                                                                                        \
-    hipLaunchKernelGGL(mh_window_kernel<VT>, dim3((unsigned)Wc), dim3(kBlk), 0, stream, fr, F0, h, k, w.src_local,   \
-                       w.edge_src, w.edge_val, tc, w.wtiles, window_offset[h], col_indices[h],                        \
+    hipLaunchKernelGGL(mh_window_kernel<VT>, dim3((unsigned)Wc), dim3(kBlk), 0, stream, fr, F0, h, k, src_local,   \
+                       w.edge_src, edge_val, tc, w.wtiles, window_offset[h], col_indices[h],                        \
                        static_cast<VT*>(values[h]), num_nodes, node_map, (int)(h + 1 == H), bitmap, grpcnt, ctr)
         if (values_dtype == GRWS_F32) GRWS_MH_WINDOWS(float);
         else if (values_dtype == GRWS_F16) GRWS_MH_WINDOWS(_Float16);
@@ -1696,36 +1712,42 @@ static int sample_blocks_impl(const int64_t* indptr, const int32_t* indices, int
         GRWS_LAUNCH_CHECK();
         if (any_t && thops[h]) {
             // the hop's slots are still in the workspace: its transposed block
+            // (once forked, every later transpose follows on the side stream:
+            // they share the sort's buffers)
+            if (h + 1 < H || ss.side != ss.main) GRWS_TRY(ss.fork_again());
+            const hipStream_t tstream = ss.side;
             const int64_t ecap = c.E[h], wcap = c.WT[h];
 #define GRWS_MH_T(KERNEL, VT, ...) hipLaunchKernelGGL(KERNEL<VT>, __VA_ARGS__)
 #define GRWS_MH_TDISPATCH(KERNEL, ...)                                                  \
     if (values_dtype == GRWS_F32) GRWS_MH_T(KERNEL, float, __VA_ARGS__);                \
     else if (values_dtype == GRWS_F16) GRWS_MH_T(KERNEL, _Float16, __VA_ARGS__);        \
     else GRWS_MH_T(KERNEL, __hip_bfloat16, __VA_ARGS__)
-            GRWS_MH_TDISPATCH(mh_tkeys_kernel, dim3(grid_for(ecap)), dim3(kBlk), 0, stream, F0, h, k,
-                              w.src_local, w.edge_val, ecap, wcap, w.tka, w.tpa, ctr);
+            GRWS_MH_TDISPATCH(mh_tkeys_kernel, dim3(grid_for(ecap)), dim3(kBlk), 0, tstream, F0, h, k,
+                              src_local, edge_val, ecap, wcap, w.tka, w.tpa, ctr);
             GRWS_LAUNCH_CHECK();
             bool alt = false;
             GRWS_TRY(radix_sort_pairs(w.tka, w.tpa, w.tkb, w.tpb, ecap, bits_for(wcap + 1), w.sort_ws, w.sort_bytes,
-                                      stream, &alt));
+                                      tstream, &alt));
             const uint64_t* sk = alt ? w.tkb : w.tka;
             const uint32_t* sp = alt ? w.tpb : w.tpa;
-            hipLaunchKernelGGL(mh_tbounds_kernel, dim3(grid_for(ecap + 1)), dim3(kBlk), 0, stream, h, sk, ecap, wcap,
+            hipLaunchKernelGGL(mh_tbounds_kernel, dim3(grid_for(ecap + 1)), dim3(kBlk), 0, tstream, h, sk, ecap, wcap,
                                w.tstart, ctr);
             GRWS_LAUNCH_CHECK();
             const unsigned tgrid = (unsigned)std::min<int64_t>((wcap + kBlk / kWave - 1) / (kBlk / kWave), 256);
-            hipLaunchKernelGGL(mh_tcount_kernel, dim3(tgrid), dim3(kBlk), 0, stream, h, k, w.tstart, sp, tc, wcap,
-                               w.wtiles, ctr);
+            hipLaunchKernelGGL(mh_tcount_kernel, dim3(tgrid), dim3(kBlk), 0, tstream, h, k, w.tstart, sp, tc, wcap,
+                               w.twtiles, ctr);
             GRWS_LAUNCH_CHECK();
-            GRWS_TRY(scan_i32_to_i64(w.wtiles, t_window_offset[h], wcap, false, w.scan_ws, w.scan_bytes, stream));
-            GRWS_MH_TDISPATCH(mh_tfill_kernel, dim3((unsigned)wcap), dim3(kBlk), 0, stream, h, k, w.tstart, sp, wcap,
-                              tc, w.src_local, w.edge_val, t_window_offset[h], t_col_indices[h], t_values[h],
+            GRWS_TRY(scan_i32_to_i64(w.twtiles, t_window_offset[h], wcap, false, w.scan_ws, w.scan_bytes,
+                                      tstream));
+            GRWS_MH_TDISPATCH(mh_tfill_kernel, dim3((unsigned)wcap), dim3(kBlk), 0, tstream, h, k, w.tstart, sp, wcap,
+                              tc, src_local, edge_val, t_window_offset[h], t_col_indices[h], t_values[h],
                               ctr);
 #undef GRWS_MH_TDISPATCH
 #undef GRWS_MH_T
             GRWS_LAUNCH_CHECK();
         }
     }
+    GRWS_TRY(ss.join());
     hipLaunchKernelGGL(mh_finish_kernel, dim3(1), dim3(64), 0, stream, ctr, counts_dev ? counts_dev : w.out, H);
     GRWS_LAUNCH_CHECK();
     if (counts_dev) return GRWS_OK;  // enqueued: the caller reads the counts after the stream's work

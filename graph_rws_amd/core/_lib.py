@@ -287,8 +287,9 @@ def check(fn: str, status: int) -> None:
 
 
 def call(fn: str, *args):
-    st = getattr(load(), fn)(*args)
-    check(fn, st)
+    st = getattr(_lib or load(), fn)(*args)
+    if st != GRWS_OK:
+        check(fn, st)
     return st
 
 
@@ -303,7 +304,9 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """t's address for a void* argument or field (a plain int: a c_void_p
+    object per argument cost a small product 2 us)."""
+    return None if t is None else t.data_ptr()
 
 
 def require_device(who: str, dev: torch.device, *tensors) -> None:
@@ -318,4 +321,8 @@ def require_device(who: str, dev: torch.device, *tensors) -> None:
 
 
 def stream_of(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    """The handle of the device's current stream (torch's own lookup, without
+    the Stream object around it)."""
+    if dev.type != "cuda":
+        return torch.cuda.current_stream(dev).cuda_stream  # raises
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)

@@ -26,6 +26,13 @@ import torch
 from ..core import csr_to_bcsr_cpu, build_spmm_plan, default_slabs
 
 
+# Longest window (slabs) that a sampled block's product takes in one work item.
+# Such a graph is multiplied once, and a plan costs it 15 launches and a
+# stream sync (190 us of a 1,024-seed mini-batch step, for one 40-slab
+# window); a wave walks a slab in well under 1 us.
+SAMPLED_SLABS = 128
+
+
 def _placed(t: torch.Tensor, device, dtype: torch.dtype) -> torch.Tensor:
     """t on `device` with `dtype`: t itself when it already is (the common
     case of arrays made on the device, e.g. sampled blocks), else a copy."""
@@ -288,7 +295,7 @@ class BCSRGraph:
             return None
         slabs = default_slabs(self.num_windows, self.num_tiles, self.tile_cols, n_cols)
         mws = getattr(self, "max_window_slabs", None)
-        if mws is not None and mws <= slabs:
+        if mws is not None and (mws <= slabs or (mws <= SAMPLED_SLABS and getattr(self, "sampled", False))):
             return None
         from ..core.ops import TensorKey
         ent = self._cache.get(("plan", slabs))

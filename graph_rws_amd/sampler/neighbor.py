@@ -144,6 +144,7 @@ class NeighborSampler:
             # at most 16 x fanout distinct columns per window
             g.max_window_slabs = (16 * k + 15) // 16
             g.fanout = k
+            g.sampled = True  # multiplied in one step, then dropped
             if tr is not None:
                 from ..core.ops import TensorKey
                 twin, tcols, tvals, tmax = tr
@@ -151,6 +152,7 @@ class NeighborSampler:
                                window_offset=twin, original_col_indices=tcols, values_condensed=tvals,
                                device=dev, num_rows=S, num_cols=16 * g.num_windows, values_dtype=self.values_dtype)
                 AT.max_window_slabs = (tmax * self.tile_cols + 15) // 16
+                AT.sampled = True
                 g._cache["T"] = (TensorKey((g.window_offset, g.original_col_indices, g.values_condensed),
                                            (g.num_cols,)), AT)
             blocks.insert(0, g)

@@ -159,8 +159,8 @@ __device__ __forceinline__ bool slot_key(const int32_t* __restrict__ cols, const
 
 // A classify kernel lists the active windows of more than kSmallCache slots;
 // two kernels share the per-window work (topk_window):
-//   * window_topk_small_kernel, one 256-thread work-group per active window,
-//     takes the others: a window's keys stay in LDS and are ranked directly;
+//   * window_topk_small_kernel, one wave per active window, takes the others
+//     (topk_wave_window): a window's keys stay in registers;
 //   * window_topk_big_kernel, 1,024-thread work-groups walking the list, on a
 //     second stream beside it (a hub window is one long work-group): keys in
 //     LDS up to kKeyCache slots, beyond that in the caller's key scratch (a
@@ -251,17 +251,17 @@ struct TopkShared {
 // slots, -1 past the sample) and its output tile count.  Every thread of the
 // work-group calls it with the same b; it leaves LDS to the caller's next
 // window only after a barrier.
-template <typename VT, int BLK, int KC, bool SMALL, int HW>
+template <typename VT, int BLK, int KC, int HW>
 __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const int64_t b, const int32_t li,
                                             const TopkArgs& a) {
     constexpr int NW = BLK / kWave;
-    constexpr int FASTMAX = SMALL ? KC : BLK;  // rank directly up to this many candidates
+    constexpr int FASTMAX = BLK;  // rank directly up to this many candidates
     // slots per thread whose loads are issued together: NB in the count pass
     // (a slot's column and 16 values), NK in the select and compaction
     // passes (one key each); more do not fit the 1,024-thread kernel's 128
     // registers without spilling
-    constexpr int NB = SMALL ? 1 : 2;
-    constexpr int NK = SMALL ? NB : 4;
+    constexpr int NB = 2;
+    constexpr int NK = 4;
     const int tid = threadIdx.x;
     const ScoreParams& p = a.p;
     const int tc = a.tc;
@@ -282,12 +282,9 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
     }
     const int64_t t0 = a.win_off[w];
     const int64_t nslots = (a.win_off[w + 1] - t0) * tc;
-    if constexpr (SMALL) {
-        if (nslots > KC) return;  // listed for the big kernel
-    }
     const bool cached = nslots <= KC;
     // keys the keys kernel computed (a listed window with scratch of its own)
-    const int64_t pre = !SMALL && li >= 0 ? a.big_goff[li] : -1;  // uniform over the work-group
+    const int64_t pre = li >= 0 ? a.big_goff[li] : -1;  // uniform over the work-group
     if (tid == 0) {
         int64_t off = -1;
         if (pre >= 0) {
@@ -314,10 +311,10 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
         }
     }
     // a listed window of more than KC slots whose keys the keys kernel
-    // computed holds only its items' cap smallest keys, packed, with their
+    // computed holds only its waves' cap smallest keys, packed, with their
     // slots beside them: the passes below scan those (nscan, set once the
     // count is known), not the window's slots
-    const bool packed = !SMALL && pre >= 0 && !cached;  // uniform over the work-group
+    const bool packed = pre >= 0 && !cached;  // uniform over the work-group
     int64_t nscan = nslots;
     // the keys of slots s + u BLK (u < NK, s + u BLK < nscan): from the LDS
     // cache or the scratch (~0: not a candidate), or recomputed
@@ -432,7 +429,7 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
         if (tid == 0) a.out_tiles[b] = (nout + tc - 1) / tc;
         return;
     }
-    if constexpr (!SMALL) {  // a small window always takes the direct ranking above
+    {
         static_assert(BLK >= kMaxCap, "the bitonic sort takes one thread per entry");
         // radix select of the cap-th smallest key (keys are distinct)
         uint64_t prefix = 0;
@@ -571,6 +568,209 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
     }
 }
 
+// The cap smallest of a wave's keys (hi word, then lo word; PER slots a lane,
+// slot lane + 64 u), in selbits.  The wanted high word is found bit by bit
+// from the top one where the least and greatest differ: a count of the
+// smaller ones is PER compares and ballots, so a selection takes at most 32
+// PER of them (and as many again among equal high words), with no barrier and
+// no memory, where ranking every key against every other took slots^2 / 64.
+// A slot that is no candidate holds ~0 in hi (below no trial value) and 0 in
+// its bit of candbits.
+template <int PER>
+__device__ __forceinline__ int wave_count_below(const uint32_t (&v)[PER], uint32_t t) {
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) c += __popcll(__ballot(v[u] < t));
+    return c;
+}
+
+// The want-th smallest (from 1) of the wave's values (~0: none) and the count
+// below it, given that there are at least `want`.
+template <int PER>
+__device__ __forceinline__ uint32_t wave_kth(const uint32_t (&v)[PER], uint32_t lo, uint32_t hi, int want, int* below) {
+    uint32_t t = lo;
+    if (lo != hi) {
+        const int top = 31 - __clz((int)(lo ^ hi));
+        t = top == 31 ? 0u : (hi >> (top + 1)) << (top + 1);
+        for (int bit = top; bit >= 0; --bit) {
+            const uint32_t trial = t | (1u << bit);
+            if (wave_count_below<PER>(v, trial) < want) t = trial;
+        }
+    }
+    *below = wave_count_below<PER>(v, t);
+    return t;
+}
+
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const uint32_t o = __shfl_xor(v, d, kWave);
+        v = o < v ? o : v;
+    }
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
+
+// Returns the number selected, min(candidates, cap); *count the candidates.
+template <int PER>
+__device__ __forceinline__ int wave_select(const uint32_t (&hi)[PER], const uint32_t (&lo)[PER], uint32_t candbits,
+                                           int cap, uint32_t* selbits, int* count) {
+    int n = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) n += __popcll(__ballot((candbits >> u) & 1u));
+    *count = n;
+    *selbits = candbits;
+    if (n <= cap) return n;  // uniform over the wave
+    uint32_t mn = ~0u, mx = 0u;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (!((candbits >> u) & 1u)) continue;
+        mn = hi[u] < mn ? hi[u] : mn;
+        mx = hi[u] > mx ? hi[u] : mx;
+    }
+    int below;
+    const uint32_t t = wave_kth<PER>(hi, wave_min_u32(mn), wave_max_u32(mx), cap, &below);
+    uint32_t sel = 0, tie = 0;
+    int ties = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const bool c = (candbits >> u) & 1u;
+        sel |= (c && hi[u] < t) ? 1u << u : 0u;
+        const bool e = c && hi[u] == t;
+        tie |= e ? 1u << u : 0u;
+        ties += __popcll(__ballot(e));
+    }
+    const int want = cap - below;  // of the ties, at least one
+    if (ties > want) {             // uniform
+        uint32_t lw[PER];
+        mn = ~0u;
+        mx = 0u;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const bool e = (tie >> u) & 1u;
+            lw[u] = e ? lo[u] : ~0u;
+            mn = e && lo[u] < mn ? lo[u] : mn;
+            mx = e && lo[u] > mx ? lo[u] : mx;
+        }
+        int lbelow;
+        const uint32_t tl = wave_kth<PER>(lw, wave_min_u32(mn), wave_max_u32(mx), want, &lbelow);
+        // equal whole keys (a column listed twice) in slot order
+        int left = want - lbelow;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const bool e = (tie >> u) & 1u;
+            const bool q = e && lo[u] == tl;
+            const uint64_t m = __ballot(q);
+            const bool in = (e && lo[u] < tl) || (q && __popcll(m & lanemask_lt()) < left);
+            left -= __popcll(m) < left ? __popcll(m) : left;
+            sel |= in ? 1u << u : 0u;
+        }
+    } else {
+        sel |= tie;
+    }
+    *selbits = sel;
+    return cap;
+}
+
+// A window of at most 64 PER slots, one wave (LDS: col and slot of its own,
+// kMaxCap each).  Most windows are small (c2: 10,434 of 10,584 have at most
+// 1,024 slots, 215 on average).  A work-group of 256 threads that ranked a
+// window's keys in LDS took 134 us for those 10,434 f32 windows, bound by its
+// compares; a wave each, selecting by bits, takes 75 us (156 MB read: 31 us at
+// 5 TB/s; the rest is the latency of a wave's few rounds of loads).
+template <typename VT, int PER>
+__device__ __forceinline__ void topk_wave_window(const TopkArgs& a, int64_t b, int32_t w, int64_t t0, int nslots,
+                                                 int32_t* __restrict__ scol, int32_t* __restrict__ sslot) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const ScoreParams& p = a.p;
+    const int tc = a.tc;
+    const int cap = a.cap, S = a.S;
+    int32_t* oc = a.out_cols + b * (int64_t)S;
+    int32_t* os = a.out_slots + b * (int64_t)S;
+    int32_t part_lo = 0, part_hi = 0;
+    bool in_part_known = false;
+    if (p.use_hacs && p.locality && p.window_part_ids && p.part_starts && p.part_ends) {
+        const int32_t pid = p.window_part_ids[w];
+        if ((int64_t)pid >= p.num_parts) {
+            if (lane == 0) atomicOr(a.err, kErrHacs);
+        } else if (pid >= 0) {
+            part_lo = p.part_starts[pid];
+            part_hi = p.part_ends[pid];
+            in_part_known = true;
+        }
+    }
+    uint32_t hi[PER], lo[PER], cand = 0;
+#pragma unroll
+    for (int u = 0; u < PER; u += 2) {  // two slots' loads in flight a lane
+        SlotRaw r[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int sl = lane + (u + q) * kWave;
+            if (sl < nslots) slot_load<VT>(a.cols, a.vals, t0, tc, sl, r[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int sl = lane + (u + q) * kWave;
+            hi[u + q] = lo[u + q] = ~0u;
+            if (sl < nslots) {
+                uint64_t k = 0;
+                if (slot_key_of(r[q], part_lo, part_hi, in_part_known, p, &k)) {
+                    hi[u + q] = (uint32_t)(k >> 32);
+                    lo[u + q] = (uint32_t)k;
+                    cand |= 1u << (u + q);
+                }
+                if (p.use_hacs && r[q].col != -1 && (r[q].col < 0 || (int64_t)r[q].col >= p.num_static_scores))
+                    atomicOr(a.err, kErrHacs);
+            }
+        }
+    }
+    uint32_t sel;
+    int count;
+    const int nsel = wave_select<PER>(hi, lo, cand, cap, &sel, &count);
+    // the kept columns in slot order, which is their ascending order in a
+    // graph whose windows list their columns ascending
+    int base = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const bool in = (sel >> u) & 1u;
+        const uint64_t m = __ballot(in);
+        if (in) {
+            const int i = base + __popcll(m & lanemask_lt());
+            scol[i] = (int32_t)lo[u];
+            sslot[i] = lane + u * kWave;
+        }
+        base += __popcll(m);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    bool up = true;
+    for (int i = lane; i + 1 < nsel; i += kWave) up = up && scol[i] < scol[i + 1];
+    const bool sorted = __ballot(!up) == 0;
+    const int nout = nsel < S ? nsel : S;
+    if (sorted) {
+        for (int i = lane; i < S; i += kWave) {
+            oc[i] = i < nout ? scol[i] : -1;
+            os[i] = i < nout ? sslot[i] : -1;
+        }
+    } else {
+        for (int i = lane; i < nsel; i += kWave) {
+            const int32_t c = scol[i];
+            int pos = 0;
+            for (int j = 0; j < nsel; ++j) pos += scol[j] < c ? 1 : 0;
+            if (pos < S) {
+                oc[pos] = c;
+                os[pos] = sslot[i];
+            }
+        }
+        for (int i = nsel + lane; i < S; i += kWave) {
+            oc[i] = -1;
+            os[i] = -1;
+        }
+    }
+    if (lane == 0) a.out_tiles[b] = (nout + tc - 1) / tc;
+}
+
 // Lists the active windows of more than kSmallCache slots (in no particular
 // order) for the big kernel; an invalid window id stays with the small
 // kernel, which reports it.  A listed window whose keys fit the scratch and
@@ -620,19 +820,19 @@ __global__ __launch_bounds__(kBlk) void window_topk_classify_kernel(TopkArgs a) 
 // scratch; every item adds its candidates to the window's count and folds
 // its least and greatest key in (atomics), as the big kernel's own count
 // pass would.  For a window of more than kKeyCache slots (which the big
-// kernel reads in place, pass after pass) an item keeps only its cap
-// smallest keys (the others cannot be among the window's cap smallest:
-// keys are distinct) and packs them, with their slots, at the window's
+// kernel reads in place, pass after pass) each wave of an item keeps only
+// its cap smallest keys (the others cannot be among the window's cap
+// smallest: keys are distinct; 60 -> 20 us of a c2 layer against ranking the
+// item's keys, and the big kernel 72 -> 30 us) and packs them, with their slots, at the window's
 // cursor.  Walks the chunks the classify kernel claimed; every work-group
 // leaves once they are done.
-static_assert(kChunk % kBlk == 0 && kChunk % 2 == 0, "whole slots per thread, key pairs in LDS");
+static_assert(kChunk % kBlk == 0, "whole slots per thread");
 template <typename VT>
 __global__ __launch_bounds__(kBlk) void window_topk_keys_kernel(TopkArgs a) {
     constexpr int PER = kChunk / kBlk;  // slots per thread and item
-    __shared__ __attribute__((aligned(16))) uint64_t skey[kChunk];
-    __shared__ int scnt;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
+    const int wbase = tid / kWave * (PER * kWave);  // the wave's slots of the item
     const ScoreParams& p = a.p;
     const int64_t claimed = *a.chunk_total;
     const int64_t total = claimed < a.chunk_cap ? claimed : a.chunk_cap;
@@ -660,12 +860,11 @@ __global__ __launch_bounds__(kBlk) void window_topk_keys_kernel(TopkArgs a) {
                 in_part_known = true;
             }
         }
-        if (tid == 0) scnt = 0;
         uint64_t kk[PER];
-        int local = 0;
+        uint32_t cand = 0;
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
-            const int64_t s = s0 + tid + u * kBlk;
+            const int64_t s = s0 + wbase + lane + u * kWave;
             kk[u] = ~0ull;
             if (s < s1) {
                 SlotRaw r;
@@ -673,81 +872,96 @@ __global__ __launch_bounds__(kBlk) void window_topk_keys_kernel(TopkArgs a) {
                 uint64_t k = 0;
                 if (slot_key_of(r, part_lo, part_hi, in_part_known, p, &k)) {
                     kk[u] = k;
-                    ++local;
+                    cand |= 1u << u;
                 }
                 if (p.use_hacs && r.col != -1 && (r.col < 0 || (int64_t)r.col >= p.num_static_scores))
                     atomicOr(a.err, kErrHacs);
             }
-            if (pack) skey[tid + u * kBlk] = kk[u];
         }
         if (pack) {
-            __syncthreads();  // scnt cleared, the item's keys in LDS
-            if (local) atomicAdd(&scnt, local);
-            __syncthreads();
-            // only the item's cap smallest keys can be among the window's cap
+            // only a wave's cap smallest keys can be among the window's cap
             // smallest (keys are distinct): the rest are dropped
-            if (scnt > a.cap) {
-                int rank[PER] = {};
-                const ulonglong2* kq = reinterpret_cast<const ulonglong2*>(skey);
-                for (int g = 0; g < kChunk / 2; ++g) {
-                    const ulonglong2 q = kq[g];
+            uint32_t hi[PER], lo[PER], sel;
+            int count;
 #pragma unroll
-                    for (int u = 0; u < PER; ++u) rank[u] += (q.x < kk[u]) + (q.y < kk[u]);
-                }
-#pragma unroll
-                for (int u = 0; u < PER; ++u)
-                    if (rank[u] >= a.cap) kk[u] = ~0ull;
+            for (int u = 0; u < PER; ++u) {
+                hi[u] = (uint32_t)(kk[u] >> 32);
+                lo[u] = (uint32_t)kk[u];
             }
+            wave_select<PER>(hi, lo, cand, a.cap, &sel, &count);
+            cand = sel;
         }
         uint64_t kmin = ~0ull, kmax = 0;
         int kept = 0;
 #pragma unroll
+        for (int u = 0; u < PER; ++u) kept += __popcll(__ballot((cand >> u) & 1u));
+        int base = 0;  // packed at the window's cursor (its count), one atomic per wave
+        if (lane == 0 && kept > 0) base = atomicAdd(&a.big_cnt[li], kept);
+        base = __shfl(base, 0, kWave);
+#pragma unroll
         for (int u = 0; u < PER; ++u) {
-            const int64_t s = s0 + tid + u * kBlk;
-            const bool keep = kk[u] != ~0ull;
+            const int64_t s = s0 + wbase + lane + u * kWave;
+            const bool keep = (cand >> u) & 1u;
             if (pack) {
-                // packed at the window's cursor (its count), one atomic per wave
                 const uint64_t m = __ballot(keep);
-                int base = 0;
-                if (lane == 0 && m) base = atomicAdd(&a.big_cnt[li], __popcll(m));
-                base = __shfl(base, 0, kWave);
                 if (keep) {
                     const int pos = base + __popcll(m & lanemask_lt());
                     gk[pos] = kk[u];
                     gs[pos] = (uint32_t)s;
                 }
+                base += __popcll(m);
             } else if (s < s1) {
                 gk[s] = kk[u];
             }
             if (keep) {
-                ++kept;
                 kmin = kk[u] < kmin ? kk[u] : kmin;
                 kmax = kk[u] > kmax ? kk[u] : kmax;
             }
         }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) kept += __shfl_xor(kept, d, kWave);
         kmin = wave_min_u64(kmin);
         kmax = wave_max_u64(kmax);
         if (lane == 0 && kept > 0) {
-            if (!pack) atomicAdd(&a.big_cnt[li], kept);
             atomicMin(&a.big_kmin[li], (unsigned long long)kmin);
             atomicMax(&a.big_kmax[li], (unsigned long long)kmax);
         }
-        if (pack) __syncthreads();  // the LDS keys are read before the next item overwrites them
     }
 }
 
+// One wave per active window of at most kSmallCache slots.
 template <typename VT>
 __global__ __launch_bounds__(kSmallBlk) void window_topk_small_kernel(TopkArgs a) {
-    __shared__ TopkShared<kSmallBlk, kSmallCache, 1> sh;
-    const int64_t b = blockIdx.x;
+    __shared__ int32_t scol[kSmallBlk / kWave][kMaxCap];
+    __shared__ int32_t sslot[kSmallBlk / kWave][kMaxCap];
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t b = (int64_t)blockIdx.x * (kSmallBlk / kWave) + wave;
     const int64_t na = a.num_active_dev ? *a.num_active_dev : a.num_active;
     if (b >= na) {  // past the device count: no tiles (the scan runs over the bound)
-        if (b < a.num_active && threadIdx.x == 0) a.out_tiles[b] = 0;
+        if (b < a.num_active && lane == 0) a.out_tiles[b] = 0;
         return;
     }
-    topk_window<VT, kSmallBlk, kSmallCache, true, 1>(sh, b, -1, a);
+    const int32_t w = a.active[b];
+    if (w < 0 || (int64_t)w >= a.num_windows) {
+        if (lane == 0) {
+            atomicOr(a.err, kErrWindow);
+            a.out_tiles[b] = 0;
+        }
+        for (int i = lane; i < a.S; i += kWave) {
+            a.out_cols[b * (int64_t)a.S + i] = -1;
+            a.out_slots[b * (int64_t)a.S + i] = -1;
+        }
+        return;
+    }
+    const int64_t t0 = a.win_off[w];
+    const int64_t nslots = (a.win_off[w + 1] - t0) * a.tc;
+    if (nslots > kSmallCache) return;  // listed for the big kernel
+    // registers for the slots there are: 4, 8 or 16 a lane (uniform)
+    if (nslots <= 4 * kWave)
+        topk_wave_window<VT, 4>(a, b, w, t0, (int)nslots, scol[wave], sslot[wave]);
+    else if (nslots <= 8 * kWave)
+        topk_wave_window<VT, 8>(a, b, w, t0, (int)nslots, scol[wave], sslot[wave]);
+    else
+        topk_wave_window<VT, kSmallCache / kWave>(a, b, w, t0, (int)nslots, scol[wave], sslot[wave]);
 }
 
 // Walks the classify kernel's list (launched after it and after the keys
@@ -758,7 +972,7 @@ __global__ __launch_bounds__(kTopkBlk) void window_topk_big_kernel(TopkArgs a) {
     __shared__ TopkShared<kTopkBlk, kKeyCache, kTopkBlk / kWave> sh;
     const int32_t n = *a.big_count;
     for (int32_t i = (int32_t)blockIdx.x; i < n; i += (int32_t)gridDim.x) {
-        topk_window<VT, kTopkBlk, kKeyCache, false, kTopkBlk / kWave>(sh, a.big_list[i], i, a);
+        topk_window<VT, kTopkBlk, kKeyCache, kTopkBlk / kWave>(sh, a.big_list[i], i, a);
         __syncthreads();
     }
 }
@@ -1186,6 +1400,7 @@ int topk_enqueue(const grws_bcsr* A, const int32_t* active_windows, int64_t num_
     // stream
     hipLaunchKernelGGL(window_topk_classify_kernel, dim3(grid_for(num_active)), dim3(kBlk), 0, stream, ta);
     GRWS_LAUNCH_CHECK();
+    const unsigned small_grid = grid_for(num_active, kSmallBlk / kWave);
     const unsigned big_grid = (unsigned)(num_active < 1024 ? num_active : 1024);
     constexpr unsigned kKeysGrid = 1024;  // the keys kernel's work-groups walk the chunks
     {
@@ -1197,7 +1412,7 @@ int topk_enqueue(const grws_bcsr* A, const int32_t* active_windows, int64_t num_
                 GRWS_LAUNCH_CHECK();
                 hipLaunchKernelGGL(window_topk_big_kernel<float>, dim3(big_grid), dim3(kTopkBlk), 0, ss.side, ta);
                 GRWS_LAUNCH_CHECK();
-                hipLaunchKernelGGL(window_topk_small_kernel<float>, dim3((unsigned)num_active), dim3(kSmallBlk), 0,
+                hipLaunchKernelGGL(window_topk_small_kernel<float>, dim3(small_grid), dim3(kSmallBlk), 0,
                                    stream, ta);
                 break;
             case GRWS_F16:
@@ -1205,7 +1420,7 @@ int topk_enqueue(const grws_bcsr* A, const int32_t* active_windows, int64_t num_
                 GRWS_LAUNCH_CHECK();
                 hipLaunchKernelGGL(window_topk_big_kernel<_Float16>, dim3(big_grid), dim3(kTopkBlk), 0, ss.side, ta);
                 GRWS_LAUNCH_CHECK();
-                hipLaunchKernelGGL(window_topk_small_kernel<_Float16>, dim3((unsigned)num_active), dim3(kSmallBlk), 0,
+                hipLaunchKernelGGL(window_topk_small_kernel<_Float16>, dim3(small_grid), dim3(kSmallBlk), 0,
                                    stream, ta);
                 break;
             default:
@@ -1215,8 +1430,8 @@ int topk_enqueue(const grws_bcsr* A, const int32_t* active_windows, int64_t num_
                 hipLaunchKernelGGL(window_topk_big_kernel<__hip_bfloat16>, dim3(big_grid), dim3(kTopkBlk), 0, ss.side,
                                    ta);
                 GRWS_LAUNCH_CHECK();
-                hipLaunchKernelGGL(window_topk_small_kernel<__hip_bfloat16>, dim3((unsigned)num_active),
-                                   dim3(kSmallBlk), 0, stream, ta);
+                hipLaunchKernelGGL(window_topk_small_kernel<__hip_bfloat16>, dim3(small_grid), dim3(kSmallBlk), 0,
+                                   stream, ta);
                 break;
         }
         GRWS_LAUNCH_CHECK();

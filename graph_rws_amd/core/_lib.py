@@ -196,6 +196,7 @@ _PROTOS = {
                                                   ctypes.c_int32, ctypes.c_int32, _vp, _vp, _vp, _vp, _vp, _vp,
                                                   _vp, _vp, _vp, ctypes.c_size_t, _vp, _vp]),
     "grws_sample_blocks_error": (ctypes.c_int, [ctypes.c_int64]),
+    "grws_count_nonzero": (ctypes.c_int, [_vp, _vp, ctypes.c_int32, ctypes.c_int32, _vp, _vp]),
     "grws_copy_ranges": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int32, _vp]),
     "grws_fill_ranges_i64": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int32, _vp]),
     "grws_probe_row_gather": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, _vp,

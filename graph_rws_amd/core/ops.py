@@ -1213,6 +1213,21 @@ def copy_and_fill(copies, fills, stream: Optional[torch.cuda.Stream] = None) -> 
     return True
 
 
+def count_nonzero(arrays) -> torch.Tensor:
+    """int64 [len(arrays)] on the arrays' device: torch.count_nonzero of each,
+    in one launch on the current stream (no sync).  Contiguous F32/F16/BF16
+    device tensors of one dtype."""
+    dev, dt = arrays[0].device, arrays[0].dtype
+    L.require_device("count_nonzero", dev, *arrays)
+    if any(t.dtype != dt or not t.is_contiguous() for t in arrays):
+        raise ValueError("count_nonzero: contiguous tensors of one dtype")
+    m = len(arrays)
+    out = torch.empty(m, dtype=torch.int64, device=dev)
+    L.call("grws_count_nonzero", (ctypes.c_void_p * m)(*[t.data_ptr() for t in arrays]),
+           (ctypes.c_int64 * m)(*[t.numel() for t in arrays]), m, L.dtype_code(dt), L.ptr(out), L.stream_of(dev))
+    return out
+
+
 def gather_rows(src: torch.Tensor, index: torch.Tensor, out: Optional[torch.Tensor] = None,
                 err: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``src.index_select(0, index)`` for a 2-D device tensor whose rows are

@@ -1104,6 +1104,50 @@ __global__ __launch_bounds__(kBlk) void seeds_dense_emit_kernel(uint32_t* __rest
     dense[w] = 0u;
 }
 
+// Nonzero values (NaN among them, -0 not) of several arrays, one row of
+// work-groups each; read 16 bytes a lane where the array is aligned.  Bound by
+// the read.
+constexpr int kCountRanges = 32;
+constexpr int kCountBlk = 1024;
+constexpr int64_t kCountGrid = 128;  // work-groups an array: one atomic each on its count (660 took 25 us)
+struct CountArgs {
+    const void* v[kCountRanges];
+    int64_t n[kCountRanges];
+    int64_t* out;
+};
+
+template <typename VT>
+__global__ __launch_bounds__(kCountBlk) void count_nonzero_kernel(CountArgs a) {
+    constexpr int V = 16 / (int)sizeof(VT);
+    __shared__ int64_t tmp[kCountBlk / kWave];
+    const int64_t n = a.n[blockIdx.y];
+    const VT* v = static_cast<const VT*>(a.v[blockIdx.y]);
+    const int64_t nv = (reinterpret_cast<uintptr_t>(v) & 15) == 0 ? n / V : 0;
+    const int64_t i0 = (int64_t)blockIdx.x * kCountBlk + threadIdx.x, step = (int64_t)gridDim.x * kCountBlk;
+    int64_t c = 0;
+    for (int64_t i = i0; i < nv; i += 4 * step) {
+        uint4 raw[4];  // four loads in flight
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            raw[q] = i + q * step < nv ? reinterpret_cast<const uint4*>(v)[i + q * step] : uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const VT* e = reinterpret_cast<const VT*>(&raw[q]);
+#pragma unroll
+            for (int k = 0; k < V; ++k) c += to_float(e[k]) != 0.0f ? 1 : 0;
+        }
+    }
+    for (int64_t i = nv * V + i0; i < n; i += step) c += to_float(v[i]) != 0.0f ? 1 : 0;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, kWave);
+    if ((threadIdx.x & (kWave - 1)) == 0) tmp[threadIdx.x / kWave] = c;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+#pragma unroll
+    for (int w = 1; w < kCountBlk / kWave; ++w) c += tmp[w];
+    if (c) atomicAdd(reinterpret_cast<unsigned long long*>(a.out + blockIdx.y), (unsigned long long)c);
+}
+
 // the batch's error flags beside its counts (an enqueued call's one word
 // the caller reads back)
 __global__ void flags_out_kernel(const int32_t* __restrict__ err, int64_t* __restrict__ out) {
@@ -1800,4 +1844,50 @@ extern "C" int grws_window_sample_layers_enqueue(const grws_bcsr* A, int64_t num
 extern "C" int grws_window_sample_layers_status(int64_t err) {
     clear_error();
     return report_topk_errors((int32_t)err, "window_sample_layers");
+}
+
+extern "C" int grws_count_nonzero(const void* const* values, const int64_t* counts, int32_t n, int32_t values_dtype,
+                                  int64_t* out, void* stream_) {
+    clear_error();
+    const hipStream_t stream = as_stream(stream_);
+    GRWS_CHECK_ARG(n >= 0, "count_nonzero: negative count");
+    if (n == 0) return GRWS_OK;
+    GRWS_CHECK_ARG(values && counts && out, "count_nonzero: null pointer");
+    if (values_dtype != GRWS_F32 && values_dtype != GRWS_F16 && values_dtype != GRWS_BF16)
+        return set_error(GRWS_E_DTYPE, "count_nonzero: unsupported values dtype %d", values_dtype);
+    int64_t most = 0;
+    for (int32_t i = 0; i < n; ++i) {
+        GRWS_CHECK_ARG(counts[i] >= 0 && (counts[i] == 0 || values[i]), "count_nonzero: bad range %d", i);
+        GRWS_CHECK_ARG(reinterpret_cast<uintptr_t>(values[i]) % dtype_size(values_dtype) == 0,
+                       "count_nonzero: range %d not aligned to its element size", i);
+        most = counts[i] > most ? counts[i] : most;
+    }
+    GRWS_TRY(fill_i64(out, n, 0, stream));
+    if (most == 0) return GRWS_OK;
+    // 4 vectors a thread and step
+    const int64_t per = (int64_t)kCountBlk * 4 * (16 / (int64_t)dtype_size(values_dtype));
+    const unsigned gx = (unsigned)std::min<int64_t>((most + per - 1) / per, kCountGrid);
+    for (int32_t base = 0; base < n; base += kCountRanges) {
+        CountArgs a{};
+        const int32_t m = std::min(n - base, (int32_t)kCountRanges);
+        for (int32_t i = 0; i < m; ++i) {
+            a.v[i] = values[base + i];
+            a.n[i] = counts[base + i];
+        }
+        a.out = out + base;
+        switch (values_dtype) {
+            case GRWS_F32:
+                hipLaunchKernelGGL(count_nonzero_kernel<float>, dim3(gx, (unsigned)m), dim3(kCountBlk), 0, stream, a);
+                break;
+            case GRWS_F16:
+                hipLaunchKernelGGL(count_nonzero_kernel<_Float16>, dim3(gx, (unsigned)m), dim3(kCountBlk), 0, stream, a);
+                break;
+            default:
+                hipLaunchKernelGGL(count_nonzero_kernel<__hip_bfloat16>, dim3(gx, (unsigned)m), dim3(kCountBlk), 0, stream,
+                                   a);
+                break;
+        }
+        GRWS_LAUNCH_CHECK();
+    }
+    return GRWS_OK;
 }

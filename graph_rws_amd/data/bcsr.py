@@ -136,13 +136,17 @@ class BCSRGraph:
     def from_components(cls, window_offset: torch.Tensor, original_col_indices: torch.Tensor,
                         values_condensed: torch.Tensor, num_rows: int, num_cols: int,
                         tile_rows: int, tile_cols: int, device: Optional[torch.device] = None,
-                        values_dtype: Optional[torch.dtype] = None) -> "BCSRGraph":
+                        values_dtype: Optional[torch.dtype] = None,
+                        num_edges: Optional[torch.Tensor] = None) -> "BCSRGraph":
         """From kernel outputs (data/bcsr.py:134-159).  num_edges is the
         count of non-zero values, as in the reference (:147), counted on the
-        values' stream now and read on first access."""
+        values' stream now and read on first access; a caller that has
+        counted them passes the 0-dim tensor."""
         if device is None:
             device = window_offset.device
-        nnz = torch.count_nonzero(values_condensed) if values_condensed.numel() > 0 else 0
+        nnz = num_edges
+        if nnz is None:
+            nnz = torch.count_nonzero(values_condensed) if values_condensed.numel() > 0 else 0
         return cls(num_nodes=int(num_rows), num_edges=nnz, tile_rows=tile_rows, tile_cols=tile_cols,
                    window_offset=window_offset, original_col_indices=original_col_indices,
                    values_condensed=values_condensed, device=device, num_rows=int(num_rows),

@@ -695,6 +695,12 @@ int grws_window_sample_layers_enqueue(const grws_bcsr* A, int64_t num_nodes, con
 /* flags, out_dev[2*num_layers] read back by the caller: GRWS_OK for 0.     */
 int grws_window_sample_layers_status(int64_t err);
 
+/* out[i] (device, int64) = the values of array i that are not zero (a
+ * sampled layer's edges, data/bcsr.py:147), for n host-listed device arrays
+ * of values_dtype.  No sync. */
+int grws_count_nonzero(const void* const* values, const int64_t* counts, int32_t n, int32_t values_dtype,
+                       int64_t* out, void* stream);
+
 size_t grws_relabel_workspace_bytes(int64_t num_frontier, int64_t num_edges);
 int grws_relabel(const int64_t* frontier, int64_t num_frontier, const int64_t* edge_src,
                  int64_t num_edges, int64_t num_nodes, int32_t* src_local, int64_t* next_frontier,

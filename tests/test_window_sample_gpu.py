@@ -6,7 +6,7 @@ import torch
 
 import oracle
 from graph_rws_amd import synth
-from graph_rws_amd.core import sample_all_layers, window_seeds
+from graph_rws_amd.core import ops, sample_all_layers, window_seeds
 from graph_rws_amd.core._lib import GrwsError
 from graph_rws_amd.data import BCSRGraph
 from graph_rws_amd.sampler import BCSRSampler
@@ -355,3 +355,18 @@ def test_bcsr_sampler_capture_option(cuda_device):
     for x, y in zip(a.sample_layers(G, seeds), b.sample_layers(G, seeds)):
         assert torch.equal(x.values_condensed.cpu(), y.values_condensed.cpu())
     assert next(iter(a._captures.values()))[1] is not cap
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+def test_count_nonzero_matches_torch(cuda_device, dt):
+    """Empty, tiny, misaligned and large arrays; NaN, infinities and -0; more
+    arrays than one launch takes."""
+    print(f"case count_nonzero {dt}", flush=True)
+    g = torch.Generator(device=cuda_device).manual_seed(3)
+    base = torch.randn(300000, generator=g, device=cuda_device).to(dt)
+    base[torch.rand(300000, generator=g, device=cuda_device) < 0.7] = 0
+    base[:6] = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0, 0.0, 1e-8], device=cuda_device).to(dt)
+    arrays = [base[o:o + n] for o, n in ((0, 0), (0, 1), (0, 7), (1, 7), (3, 1000), (0, 4096), (5, 262144), (0, 300000))]
+    arrays += [base[i:i + 50] for i in range(40)]
+    got = ops.count_nonzero(arrays)
+    assert got.tolist() == [int(torch.count_nonzero(a)) for a in arrays]

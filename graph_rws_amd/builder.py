@@ -60,9 +60,11 @@ def _build(row_ptr, rows, cols, values, nnz: int, num_rows: int, num_cols: int, 
     ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
     T = ctypes.c_int64()
     stream = L.stream_of(dev)
-    L.call("grws_bcsr_build_count", L.ptr(row_ptr), L.ptr(rows), L.ptr(cols), L.ptr(values), nnz,
-           num_rows, num_cols, tile_cols, int(transpose), L.ptr(win), L.ptr(ws), wsb,
-           ctypes.byref(T), stream)
+    sizes = (nnz, num_rows, num_cols, tile_cols, int(transpose), L.ptr(win), L.ptr(ws), wsb, ctypes.byref(T), stream)
+    if rows is not None and rows.dtype == torch.int64:
+        L.call("grws_bcsr_build_count_i64", L.ptr(rows), L.ptr(cols), L.ptr(values), *sizes)
+    else:
+        L.call("grws_bcsr_build_count", L.ptr(row_ptr), L.ptr(rows), L.ptr(cols), L.ptr(values), *sizes)
     return (win,) + _fill(nnz, num_rows, num_cols, tile_cols, transpose, win, T.value, values_dtype, ws, wsb, stream)
 
 
@@ -100,8 +102,10 @@ def coo_to_bcsr_device(num_rows: int, num_cols: int, rows: torch.Tensor, cols: t
     BCSR on the device, in one sort."""
     dev = rows.device
     L.require_device("coo_to_bcsr_device", dev)  # the other inputs are moved to dev below
-    r = _i32(rows, dev)
-    c = _i32(cols, dev)
+    if rows.dtype == cols.dtype == torch.int64 and cols.device == dev:
+        r, c = rows.contiguous(), cols.contiguous()  # the build reads them as they are
+    else:
+        r, c = _i32(rows, dev), _i32(cols, dev)
     va = None if values is None else values.to(dev, torch.float32).contiguous()
     if r.numel() != c.numel():
         raise ValueError("rows and cols differ in length")

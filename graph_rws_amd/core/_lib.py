@@ -117,6 +117,9 @@ _PROTOS = {
     "grws_bcsr_build_count": (ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64,
                                              ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _vp,
                                              _vp, ctypes.c_size_t, _c_i64p, _vp]),
+    "grws_bcsr_build_count_i64": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+                                                 ctypes.c_int32, ctypes.c_int32, _vp, _vp, ctypes.c_size_t,
+                                                 _c_i64p, _vp]),
     "grws_bcsr_build_fill": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                             ctypes.c_int32, ctypes.c_int32, _vp, ctypes.c_int64,
                                             _vp, _vp, ctypes.c_int32, _vp, ctypes.c_size_t, _vp]),

@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kBlk = 256;
 
-enum : int32_t { kErrRow = 1, kErrCol = 2, kErrRowPtr = 4 };
+enum : int32_t { kErrRow = kErrEdgeRow, kErrCol = kErrEdgeCol, kErrRowPtr = 4 };
 
 // Bits needed to hold every value in [0, x).
 inline int bits_for(int64_t x) {
@@ -119,17 +119,6 @@ __global__ void check_row_ptr_kernel(const int64_t* __restrict__ row_ptr, int64_
     if (bad) atomicOr(err, kErrRowPtr);
 }
 
-// Row of edge e in a CSR: the largest r with row_ptr[r] <= e.
-__device__ __forceinline__ int64_t csr_row_of(const int64_t* __restrict__ row_ptr, int64_t num_rows, int64_t e) {
-    int64_t lo = 0, hi = num_rows - 1;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi + 1) >> 1;
-        if (row_ptr[mid] <= e) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // An edge's sort key from its window-row wr (the BCSR row) and column cc.
 // wbits == 0: (window, column, row-in-window), the global sort's key.
 // wbits > 0 (a multiple of 8): window | row-in-window << wbits | column <<
@@ -137,18 +126,20 @@ __device__ __forceinline__ int64_t csr_row_of(const int64_t* __restrict__ row_pt
 // equal edges have equal keys, so a stable sort keeps duplicates in input
 // order.
 __device__ __forceinline__ uint64_t edge_key(int64_t wr, int64_t cc, int cbits, int wbits) {
-    if (wbits) return (uint64_t)(wr >> 4) | ((uint64_t)(wr & 15) << wbits) | ((uint64_t)cc << (wbits + 4));
+    if (wbits) return window_key(wr, cc, wbits);
     return ((uint64_t)(wr >> 4) << (cbits + 4)) | ((uint64_t)cc << 4) | (uint64_t)(wr & 15);
 }
 
-__global__ void build_keys_kernel(const int64_t* __restrict__ row_ptr, const int32_t* __restrict__ rows,
-                                  const int32_t* __restrict__ cols, const float* __restrict__ vals, int64_t n,
+// A COO's keys (int64 ids modulo 2^32, as a cast to int32 takes them).
+template <typename IT>
+__global__ void build_keys_kernel(const IT* __restrict__ rows, const IT* __restrict__ cols,
+                                  const float* __restrict__ vals, int64_t n,
                                   int64_t num_rows, int64_t num_cols, int transpose, int cbits, int wbits,
                                   uint64_t* __restrict__ keys, uint32_t* __restrict__ pay, int32_t* __restrict__ err) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    int64_t r = rows ? (int64_t)rows[i] : csr_row_of(row_ptr, num_rows, i);
-    int64_t c = cols[i];
+    int64_t r = (int32_t)rows[i];
+    int64_t c = (int32_t)cols[i];
     int32_t e = 0;
     if (r < 0 || r >= num_rows) { e |= kErrRow; r = 0; }
     if (c < 0 || c >= num_cols) { e |= kErrCol; c = 0; }
@@ -1398,9 +1389,11 @@ extern "C" size_t grws_bcsr_build_workspace_bytes(int64_t nnz, int64_t num_rows,
 }
 
 // The count phase after its checks.  emit_keys(wbits) writes the nnz edge
-// keys of that layout (edge_key) and their values to w.ka / w.va.
+// keys of that layout (edge_key) and their values to w.ka / w.va.  coo: the
+// edge list, for a window-major sort whose first pass makes the keys itself
+// (115M edges: 0.63 ms and 2.7 GB less than writing and reading them).
 template <typename EmitKeys>
-static int build_count(const BuildShape& s, BuildWs& w, const int64_t* row_ptr, const int32_t* cols,
+static int build_count(const CooEdges* coo, const BuildShape& s, BuildWs& w, const int64_t* row_ptr, const int32_t* cols,
                        const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols, int32_t tile_cols,
                        int32_t transpose, int64_t* window_offset, int64_t* num_tiles_out, hipStream_t stream,
                        EmitKeys emit_keys) {
@@ -1438,8 +1431,14 @@ static int build_count(const BuildShape& s, BuildWs& w, const int64_t* row_ptr, 
         per_window = (h[0] & kErrRowPtr) == 0 && h[3] == 0;
         nbig = h[1];
     } else if (nnz > 0 && s.C <= ((int64_t)1 << 27)) {
-        GRWS_TRY(emit_keys(kwbits));
-        GRWS_TRY(radix_sort_pairs(w.ka, w.va, w.kb, w.vb, nnz, kwbits, w.sort_ws, w.sort_bytes, stream, &kalt));
+        if (coo && radix_sorts_edges(nnz)) {
+            CooEdges e = *coo;
+            e.wbits = kwbits;
+            GRWS_TRY(radix_sort_edges(e, w.ka, w.va, w.kb, w.vb, nnz, kwbits, w.sort_ws, w.sort_bytes, stream, &kalt));
+        } else {
+            GRWS_TRY(emit_keys(kwbits));
+            GRWS_TRY(radix_sort_pairs(w.ka, w.va, w.kb, w.vb, nnz, kwbits, w.sort_ws, w.sort_bytes, stream, &kalt));
+        }
         if (nnz >= kBoundsSearch)
             hipLaunchKernelGGL(keyed_bounds_search_kernel, dim3(grid_for(s.W, 64)), dim3(64), 0, stream,
                                kalt ? w.kb : w.ka, nnz, ((uint64_t)1 << kwbits) - 1, s.W, w.wstart, w.wend);
@@ -1553,12 +1552,12 @@ static int build_count(const BuildShape& s, BuildWs& w, const int64_t* row_ptr, 
     return GRWS_OK;
 }
 
-extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows, const int32_t* cols,
-                                     const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols,
-                                     int32_t tile_cols, int32_t transpose, int64_t* window_offset, void* workspace,
-                                     size_t workspace_bytes, int64_t* num_tiles_out, void* stream_) {
-    clear_error();
-    hipStream_t stream = as_stream(stream_);
+// ids64: rows and cols are int64 (COO input only)
+static int build_count_checked(const int64_t* row_ptr, const void* rows, const void* cols_, bool ids64,
+                               const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols,
+                               int32_t tile_cols, int32_t transpose, int64_t* window_offset, void* workspace,
+                               size_t workspace_bytes, int64_t* num_tiles_out, hipStream_t stream) {
+    const int32_t* cols = ids64 ? nullptr : static_cast<const int32_t*>(cols_);
     GRWS_TRY(refuse_capture(stream, "bcsr_build_count"));
     GRWS_CHECK_ARG(nnz >= 0 && num_rows >= 0 && num_cols >= 0, "bcsr_build: negative size");
     GRWS_CHECK_ARG(num_rows <= INT32_MAX && num_cols <= INT32_MAX, "bcsr_build: dimensions exceed int32 ids");
@@ -1567,7 +1566,7 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
     GRWS_CHECK_ARG(window_offset && num_tiles_out, "bcsr_build: null output");
     GRWS_CHECK_ARG(row_ptr == nullptr || rows == nullptr, "bcsr_build: pass only one of row_ptr and rows");
     if (nnz > 0) GRWS_CHECK_ARG(row_ptr != nullptr || rows != nullptr, "bcsr_build: pass row_ptr or rows");
-    if (nnz > 0) GRWS_CHECK_ARG(cols != nullptr, "bcsr_build: null cols");
+    if (nnz > 0) GRWS_CHECK_ARG(cols_ != nullptr, "bcsr_build: null cols");
     if (row_ptr) GRWS_CHECK_ARG(num_rows > 0 || nnz == 0, "bcsr_build: edges without rows");
     BuildShape s = build_shape(nnz, num_rows, num_cols, transpose);
     Carver cv(workspace, workspace_bytes);
@@ -1575,11 +1574,17 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
     carve_build(cv, s, &w);
     if (!cv.ok) return set_error(GRWS_E_CAPACITY, "bcsr_build: workspace too small (%zu < %zu)", workspace_bytes, cv.used);
 
-    return build_count(s, w, row_ptr, cols, values, nnz, num_rows, num_cols, tile_cols, transpose, window_offset,
+    const CooEdges coo{rows, cols_, values, num_rows, num_cols, transpose, 0, ids64 ? 1 : 0, w.err};
+    return build_count(rows ? &coo : nullptr, s, w, row_ptr, cols, values, nnz, num_rows, num_cols, tile_cols, transpose, window_offset,
                        num_tiles_out, stream, [&](int wbits) -> int {
-        if (rows) {
-            hipLaunchKernelGGL(build_keys_kernel, dim3(grid_for(nnz)), dim3(kBlk), 0, stream, row_ptr, rows, cols,
-                               values, nnz, num_rows, num_cols, (int)transpose, s.cbits, wbits, w.ka, w.va, w.err);
+        if (rows && ids64) {
+            hipLaunchKernelGGL(build_keys_kernel<int64_t>, dim3(grid_for(nnz)), dim3(kBlk), 0, stream,
+                               static_cast<const int64_t*>(rows), static_cast<const int64_t*>(cols_), values, nnz,
+                               num_rows, num_cols, (int)transpose, s.cbits, wbits, w.ka, w.va, w.err);
+        } else if (rows) {
+            hipLaunchKernelGGL(build_keys_kernel<int32_t>, dim3(grid_for(nnz)), dim3(kBlk), 0, stream,
+                               static_cast<const int32_t*>(rows), cols, values, nnz, num_rows, num_cols,
+                               (int)transpose, s.cbits, wbits, w.ka, w.va, w.err);
         } else {
             // every edge lies in some row's range (check_row_ptr_kernel flags
             // a row pointer that does not cover [0, nnz) exactly)
@@ -1591,6 +1596,24 @@ extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows
         GRWS_LAUNCH_CHECK();
         return GRWS_OK;
     });
+}
+
+extern "C" int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows, const int32_t* cols,
+                                     const float* values, int64_t nnz, int64_t num_rows, int64_t num_cols,
+                                     int32_t tile_cols, int32_t transpose, int64_t* window_offset, void* workspace,
+                                     size_t workspace_bytes, int64_t* num_tiles_out, void* stream_) {
+    clear_error();
+    return build_count_checked(row_ptr, rows, cols, false, values, nnz, num_rows, num_cols, tile_cols, transpose,
+                               window_offset, workspace, workspace_bytes, num_tiles_out, as_stream(stream_));
+}
+
+extern "C" int grws_bcsr_build_count_i64(const int64_t* rows, const int64_t* cols, const float* values, int64_t nnz,
+                                         int64_t num_rows, int64_t num_cols, int32_t tile_cols, int32_t transpose,
+                                         int64_t* window_offset, void* workspace, size_t workspace_bytes,
+                                         int64_t* num_tiles_out, void* stream_) {
+    clear_error();
+    return build_count_checked(nullptr, rows, cols, true, values, nnz, num_rows, num_cols, tile_cols, transpose,
+                               window_offset, workspace, workspace_bytes, num_tiles_out, as_stream(stream_));
 }
 
 extern "C" int grws_bcsr_build_fill(int64_t nnz, int64_t num_rows, int64_t num_cols, int32_t tile_cols,
@@ -1895,7 +1918,7 @@ extern "C" int grws_bcsr_transpose_count(const grws_bcsr* A, int64_t num_cols, i
         // the per-tile counts are spent (toff holds their scan)
         GRWS_TRY(launch_tile_windows(A, twin, stream));
     }
-    return build_count(s, w, nullptr, nullptr, nullptr, nnz, rows, num_cols, tile_cols, 1, window_offset,
+    return build_count(nullptr, s, w, nullptr, nullptr, nullptr, nnz, rows, num_cols, tile_cols, 1, window_offset,
                        num_tiles_out, stream, [&](int wbits) -> int {
         return launch_tile_emit<true>(A, num_cols, twin, toff, nullptr, nullptr, nullptr, s.cbits, wbits, w.ka, w.va,
                                       stream);

@@ -131,8 +131,64 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t ntiles) {
     return (blockIdx.x >> 3) < per ? t : ntiles;
 }
 
-__global__ __launch_bounds__(kRbBlock) void radix_hist_big_kernel(const uint64_t* __restrict__ keys, int64_t n,
-                                                                  int shift, int64_t ntiles,
+// What a pass reads: sorted pairs, or (the first pass of a COO build) the
+// edge list itself, its keys made on the fly.  digit(): what the count needs
+// of element i; get(): its key and payload.
+struct PairSrc {
+    const uint64_t* keys;
+    const uint32_t* vals;
+    __device__ __forceinline__ uint64_t digit(int64_t i) const { return keys[i]; }
+    using Raw = uint64_t;
+    __device__ __forceinline__ Raw load(int64_t i) const { return keys[i]; }
+    __device__ __forceinline__ uint64_t key(Raw r, int32_t*) const { return r; }
+    __device__ __forceinline__ void report(int32_t) const {}
+    __device__ __forceinline__ uint32_t pay(int64_t i) const { return vals[i]; }
+    __device__ __forceinline__ bool has_pay() const { return vals != nullptr; }
+};
+
+// IT: int32_t, or int64_t ids taken modulo 2^32 as a cast to int32 takes them.
+template <typename IT>
+struct CooSrc {
+    CooEdges e;
+    struct Raw {
+        int32_t r, c;
+    };
+    __device__ __forceinline__ Raw load(int64_t i) const {
+        return Raw{(int32_t) static_cast<const IT*>(e.rows)[i], (int32_t) static_cast<const IT*>(e.cols)[i]};
+    }
+    // a bad id counts as id 0, here as in digit()
+    __device__ __forceinline__ int64_t row(int32_t r, int32_t* bad) const {
+        if (r >= 0 && r < e.num_rows) return r;
+        *bad |= kErrEdgeRow;
+        return 0;
+    }
+    __device__ __forceinline__ int64_t col(int32_t c, int32_t* bad) const {
+        if (c >= 0 && c < e.num_cols) return c;
+        *bad |= kErrEdgeCol;
+        return 0;
+    }
+    // the low bits of the key: the window
+    __device__ __forceinline__ uint64_t digit(int64_t i) const {
+        int32_t bad = 0;
+        return (uint64_t)((e.transpose ? col((int32_t) static_cast<const IT*>(e.cols)[i], &bad)
+                                       : row((int32_t) static_cast<const IT*>(e.rows)[i], &bad)) >>
+                          4);
+    }
+    __device__ __forceinline__ uint64_t key(Raw q, int32_t* bad) const {
+        const int64_t r = row(q.r, bad), c = col(q.c, bad);
+        return e.transpose ? window_key(c, r, e.wbits) : window_key(r, c, e.wbits);
+    }
+    __device__ __forceinline__ void report(int32_t bad) const {
+        if (bad) atomicOr(e.err, bad);
+    }
+    __device__ __forceinline__ uint32_t pay(int64_t i) const {
+        return e.vals ? __float_as_uint(e.vals[i]) : 0x3f800000u;  // 1.0f when no values are given
+    }
+    __device__ __forceinline__ bool has_pay() const { return true; }
+};
+
+template <typename Src>
+__global__ __launch_bounds__(kRbBlock) void radix_hist_big_kernel(Src src, int64_t n, int shift, int64_t ntiles,
                                                                   int32_t* __restrict__ counts) {
     __shared__ int32_t h[kRbWaves][256];
     const int64_t t = xcd_tile(ntiles);
@@ -145,7 +201,7 @@ __global__ __launch_bounds__(kRbBlock) void radix_hist_big_kernel(const uint64_t
 #pragma unroll
     for (int it = 0; it < kRbItems; ++it) {
         const int64_t i = base + it * kRbBlock + tid;
-        k[it] = i < n ? keys[i] : 0;
+        k[it] = i < n ? src.digit(i) : 0;
     }
 #pragma unroll
     for (int it = 0; it < kRbItems; ++it)
@@ -159,9 +215,8 @@ __global__ __launch_bounds__(kRbBlock) void radix_hist_big_kernel(const uint64_t
     }
 }
 
-__global__ __launch_bounds__(kRbBlock) void radix_scatter_big_kernel(const uint64_t* __restrict__ kin,
-                                                                     const uint32_t* __restrict__ vin, int64_t n,
-                                                                     int shift, int64_t ntiles,
+template <typename Src>
+__global__ __launch_bounds__(kRbBlock) void radix_scatter_big_kernel(Src src, int64_t n, int shift, int64_t ntiles,
                                                                      const int64_t* __restrict__ offsets,
                                                                      uint64_t* __restrict__ kout,
                                                                      uint32_t* __restrict__ vout) {
@@ -177,18 +232,23 @@ __global__ __launch_bounds__(kRbBlock) void radix_scatter_big_kernel(const uint6
     uint64_t k[kRbItems];
     uint32_t v[kRbItems];
     uint32_t place[kRbItems];
+    typename Src::Raw raw[kRbItems] = {};
 #pragma unroll
-    for (int it = 0; it < kRbItems; ++it) {
+    for (int it = 0; it < kRbItems; ++it) {  // every load issued before the first is used
         const int64_t i = base + it * kWave;
-        k[it] = i < n ? kin[i] : 0;
+        if (i < n) raw[it] = src.load(i);
     }
-    if (vin) {
+    if (src.has_pay()) {
 #pragma unroll
         for (int it = 0; it < kRbItems; ++it) {
             const int64_t i = base + it * kWave;
-            v[it] = i < n ? vin[i] : 0;
+            v[it] = i < n ? src.pay(i) : 0;
         }
     }
+    int32_t bad = 0;
+#pragma unroll
+    for (int it = 0; it < kRbItems; ++it) k[it] = base + it * kWave < n ? src.key(raw[it], &bad) : 0;
+    src.report(bad);
     __syncthreads();
     // rank among the wave's keys of the same digit, in index order
     volatile int32_t* mine = wcnt[wave];
@@ -249,7 +309,7 @@ __global__ __launch_bounds__(kRbBlock) void radix_scatter_big_kernel(const uint6
             kout[pos[it]] = key;
         }
     }
-    if (!vin) return;  // uniform
+    if (!src.has_pay()) return;  // uniform
     __syncthreads();
     uint32_t* pstage = reinterpret_cast<uint32_t*>(stage);
 #pragma unroll
@@ -279,8 +339,8 @@ size_t radix_sort_workspace_bytes(int64_t n) {
     return s.used;
 }
 
-int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits,
-                     void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt) {
+static int sort_passes(const CooEdges* coo, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
+                       int64_t n, int bits, void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt) {
     *result_in_alt = false;
     if (n <= 1 || bits <= 0) return GRWS_OK;
     if (bits > 64) bits = 64;
@@ -303,17 +363,31 @@ int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_
     bool alt = false;
     for (int shift = 0; shift < bits; shift += 8) {
         const unsigned bgrid = (unsigned)((ntiles + 7) / 8 * 8);
-        if (big)
-            hipLaunchKernelGGL(radix_hist_big_kernel, dim3(bgrid), dim3(kRbBlock), 0, stream, ka, n, shift, ntiles,
-                               counts);
+        const PairSrc pairs{ka, va};
+        const bool first = coo != nullptr && shift == 0;
+        if (first && coo->ids64)
+            hipLaunchKernelGGL(radix_hist_big_kernel<CooSrc<int64_t>>, dim3(bgrid), dim3(kRbBlock), 0, stream,
+                               CooSrc<int64_t>{*coo}, n, shift, ntiles, counts);
+        else if (first)
+            hipLaunchKernelGGL(radix_hist_big_kernel<CooSrc<int32_t>>, dim3(bgrid), dim3(kRbBlock), 0, stream,
+                               CooSrc<int32_t>{*coo}, n, shift, ntiles, counts);
+        else if (big)
+            hipLaunchKernelGGL(radix_hist_big_kernel<PairSrc>, dim3(bgrid), dim3(kRbBlock), 0, stream, pairs, n,
+                               shift, ntiles, counts);
         else
             hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)ntiles), dim3(kRsBlock), 0, stream, ka, n, shift,
                                ntiles, iters, counts);
         GRWS_LAUNCH_CHECK();
         GRWS_TRY(scan_i32_to_i64(counts, offsets, 256 * ntiles, false, scan_ws, scan_bytes, stream));
-        if (big)
-            hipLaunchKernelGGL(radix_scatter_big_kernel, dim3(bgrid), dim3(kRbBlock), 0, stream, ka, va, n, shift,
-                               ntiles, offsets, kb, vb);
+        if (first && coo->ids64)
+            hipLaunchKernelGGL(radix_scatter_big_kernel<CooSrc<int64_t>>, dim3(bgrid), dim3(kRbBlock), 0, stream,
+                               CooSrc<int64_t>{*coo}, n, shift, ntiles, offsets, kb, vb);
+        else if (first)
+            hipLaunchKernelGGL(radix_scatter_big_kernel<CooSrc<int32_t>>, dim3(bgrid), dim3(kRbBlock), 0, stream,
+                               CooSrc<int32_t>{*coo}, n, shift, ntiles, offsets, kb, vb);
+        else if (big)
+            hipLaunchKernelGGL(radix_scatter_big_kernel<PairSrc>, dim3(bgrid), dim3(kRbBlock), 0, stream, pairs, n,
+                               shift, ntiles, offsets, kb, vb);
         else
             hipLaunchKernelGGL(radix_scatter_kernel, dim3((unsigned)ntiles), dim3(kRsBlock), 0, stream, ka, va, n,
                                shift, ntiles, iters, offsets, kb, vb);
@@ -324,6 +398,18 @@ int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_
     }
     *result_in_alt = alt;
     return GRWS_OK;
+}
+
+int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits,
+                     void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt) {
+    return sort_passes(nullptr, keys, vals, keys_alt, vals_alt, n, bits, ws, ws_bytes, stream, result_in_alt);
+}
+
+bool radix_sorts_edges(int64_t n) { return n >= kRsBigKeys && n <= (int64_t)UINT32_MAX; }
+
+int radix_sort_edges(const CooEdges& coo, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
+                     int64_t n, int bits, void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt) {
+    return sort_passes(&coo, keys, vals, keys_alt, vals_alt, n, bits, ws, ws_bytes, stream, result_in_alt);
 }
 
 }  // namespace grws

@@ -341,6 +341,13 @@ int grws_bcsr_build_count(const int64_t* row_ptr, const int32_t* rows, const int
                           void* workspace, size_t workspace_bytes, int64_t* num_tiles_out,
                           void* stream);
 
+/* The count phase of a COO whose ids are int64 (taken modulo 2^32, as a cast
+ * to int32 takes them): same result as casting them first. */
+int grws_bcsr_build_count_i64(const int64_t* rows, const int64_t* cols, const float* values, int64_t nnz,
+                              int64_t num_rows, int64_t num_cols, int32_t tile_cols, int32_t transpose,
+                              int64_t* window_offset, void* workspace, size_t workspace_bytes,
+                              int64_t* num_tiles_out, void* stream);
+
 /* Phase 2.  Same sizes and the workspace phase 1 left (unmodified); fills
  * col_indices [num_tiles*tile_cols] (-1 padding) and values
  * [num_tiles*16*tile_cols] of values_dtype (round to nearest even). */

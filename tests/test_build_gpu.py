@@ -677,3 +677,32 @@ def test_loaded_edges_equal_the_csr_route(cuda_device, tc, vdt, n, m, nnz):
                 for a in ("window_offset", "original_col_indices", "values_condensed"):
                     assert torch.equal(getattr(ref, a), getattr(got, a)), a
                 assert (ref.num_edges, ref.num_rows, ref.num_cols) == (got.num_edges, got.num_rows, got.num_cols)
+
+
+@pytest.mark.parametrize("nnz", [(1 << 20) - 1, 1 << 20, (1 << 20) + 8191])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_edge_list_sort_makes_its_keys(cuda_device, nnz, transpose):
+    """The first sort pass over an edge list (2^20 edges and more) against the
+    keys written first (below), with int32 and int64 ids, int64 ids past 32
+    bits (taken modulo 2^32), without values, and a bad id flagged."""
+    print(f"case edge list sort nnz={nnz} transpose={transpose}", flush=True)
+    n, m = 40000, 33333
+    g = torch.Generator(device=cuda_device).manual_seed(nnz)
+    r = torch.randint(0, n, (nnz,), generator=g, device=cuda_device)
+    c = torch.randint(0, m, (nnz,), generator=g, device=cuda_device)
+    v = torch.randn(nnz, generator=g, device=cuda_device)
+    # the same matrix through the CSR route (no edge-list sort)
+    _, rp, ci, va = builder.coo_to_csr_device(n, m, r, c, v)
+    ref = builder.csr_to_bcsr_device(n, m, rp, ci, va, tile_cols=16, values_dtype=torch.float16, transpose=transpose)
+    for rr, cc in ((r.int(), c.int()), (r, c), (r + (1 << 32), c - (1 << 32))):
+        got = builder.coo_to_bcsr_device(n, m, rr, cc, v, tile_cols=16, values_dtype=torch.float16,
+                                         transpose=transpose)
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b)
+    ones = builder.coo_to_bcsr_device(n, m, r, c, None, transpose=transpose)
+    assert torch.equal(ones[0], ref[0]) and torch.equal(ones[1], ref[1]) and set(ones[2].unique().tolist()) <= {0.0, 1.0}
+    for bad_r, bad_c in ((n, 0), (-1, 0), (0, m), (0, -7)):
+        rb, cb = r.clone(), c.clone()
+        rb[nnz // 2], cb[nnz // 2] = bad_r, bad_c
+        with pytest.raises(GrwsError, match="range"):
+            builder.coo_to_bcsr_device(n, m, rb, cb, v, transpose=transpose)

@@ -127,8 +127,8 @@ def bench_build(g, dev, cpu: bool, reps: int = 5, cfg: str = "c3") -> dict:
          "ms": round(1e3 * t_fwd, 3), "edges_per_s": round(nnz / t_fwd, 1),
          "path": "window by window" if per_window else "global radix sort", "radix_passes": passes,
          "transpose_ms": round(1e3 * t_tr, 3),
-         "transpose_how": "BCSR(A) -> COO -> BCSR(A^T): the COO grouped by window (radix sort over the window "
-                          "bits), then built window by window",
+         "transpose_how": "BCSR(A) -> BCSR(A^T): the tiles' edges written as sort keys, grouped by window (radix "
+                          "sort over the window bits), then built window by window",
          "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                       "frac": round(gbs / HBM_PEAK_GBS, 4), "bytes": int(b_alg),
                       "note": "algorithmic bytes of the path taken: the CSR read, the BCSR written once, and "

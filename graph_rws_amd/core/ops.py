@@ -1618,9 +1618,14 @@ def gemm_tn(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype = torch.flo
 
 def gemm_tn_f32_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether gemm_tn_f32 takes these operands: F32 2-D CUDA tensors with
-    equal row counts and unit column stride (any widths and row strides)."""
+    equal row counts, at most 65,536 columns, unit column stride and rows
+    that do not overlap (any row stride of at least the width; an expanded
+    tensor's is 0), and with storage (a batch of gradients under vmap has
+    none)."""
     return (a.is_cuda and b.is_cuda and a.dim() == 2 and b.dim() == 2 and a.dtype == torch.float32
-            and b.dtype == torch.float32 and a.shape[0] == b.shape[0] and a.stride(1) == 1 and b.stride(1) == 1)
+            and b.dtype == torch.float32 and a.shape[0] == b.shape[0] and a.stride(1) == 1 and b.stride(1) == 1
+            and a.shape[1] <= min(65536, a.stride(0)) and b.shape[1] <= min(65536, b.stride(0))
+            and torch._C._has_storage(a) and torch._C._has_storage(b))
 
 
 def gemm_tn_f32(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:

@@ -113,3 +113,37 @@ def test_gemm_tn_f32_matches_float64(cuda_device, K, M, N):
     assert torch.equal(C, gemm_tn_f32(A, wide[:, :N]))
     wide[:, 1:N + 1] = B  # a misaligned start
     assert torch.equal(C, gemm_tn_f32(A, wide[:, 1:N + 1]))
+
+
+def test_tall_f32_weight_grad_of_expanded_and_batched_operands(cuda_device):
+    """Operands the f32 kernel does not take (rows that share memory,
+    gradients batched by vmap) go to the library's product."""
+    from graph_rws_amd.layers.layer import F32_TN_ROWS, _weight_grad
+    n = F32_TN_ROWS + 3
+    gen = torch.Generator(device=cuda_device).manual_seed(5)
+    x = torch.randn(n, 24, generator=gen, device=cuda_device)
+    g = torch.randn(n, 9, generator=gen, device=cuda_device)
+    ones = torch.ones(1, 24, device=cuda_device).expand(n, 24)
+
+    class Product(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, w):
+            ctx.save_for_backward(x)
+            return x @ w
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None, _weight_grad(ctx.saved_tensors[0], grad.contiguous())
+
+    def close(c, a, b):  # n f32 sums
+        bound = a.double().abs().t() @ b.double().abs()
+        assert bool(((c.double() - a.double().t() @ b.double()).abs() <= n * 2.0 ** -24 * bound).all())
+
+    with torch.no_grad():
+        close(_weight_grad(ones, g), ones, g)
+        close(_weight_grad(x, g), x, g)
+    w = torch.randn(24, 9, generator=gen, device=cuda_device, requires_grad=True)
+    both = torch.stack([g, 2 * g])
+    dw, = torch.autograd.grad(Product.apply(x, w), w, both, is_grads_batched=True)
+    close(dw[0], x, g)
+    close(dw[1], x, 2 * g)

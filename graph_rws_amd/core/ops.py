@@ -1628,6 +1628,14 @@ def gemm_tn_f32_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
             and torch._C._has_storage(a) and torch._C._has_storage(b))
 
 
+def gemm_tn_f32_tiles(m: int, n: int) -> int:
+    """Output tiles of gemm_tn_f32 for [m, n]: each side in tiles of 32, 64 or
+    128 columns, the first that covers it (f32_shape in csrc/gemm_tn.hip)."""
+    def side(c):
+        return -(-c // (32 if c <= 32 else 64 if c <= 64 else 128))
+    return side(m) * side(n)
+
+
 def gemm_tn_f32(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T @ b for F32 a [K, M], b [K, N] (split over K, deterministic)."""
     if not gemm_tn_f32_supported(a, b):

@@ -37,11 +37,23 @@ FUSED_SELF = True
 PAD_AGGREGATE = True
 
 
-# Rows from which an f32 weight gradient takes the split-K kernel.  Measured
-# (us, library / kernel): 128 x 256 at 4,096 rows 26 / 32, at 16,384 rows
-# 99 / 31, at 169,343 rows 440 / 116; 608 x 256 at 4,096 rows 27 / 41, at
-# 16,384 rows 107 / 69; 1433 x 16 at 4,096 rows 20 / 21, at 16,384 55 / 38.
+# When an f32 weight gradient takes the split-K kernel: from F32_TN_ROWS rows,
+# and up to F32_TN_TILES output tiles (ops.gemm_tn_f32_tiles), or F32_TN_RAGGED
+# when rows are not whole 16-byte vectors (four loads for one).  The kernel
+# wins where the output is too small for the library to fill the device; with
+# more tiles the library does without partial sums.  Measured (us, library /
+# kernel; tiles in brackets).  Rows: 128 x 256 [2] at 4,096 rows 26 / 32, at
+# 16,384 rows 99 / 31, at 169,343 rows 440 / 116; 608 x 256 [10] at 4,096 rows
+# 27 / 41, at 16,384 107 / 69.  Tiles, at 16,384 / 65,536 / 169,343 rows:
+# 1024 x 256 [16] 104 / 89, 597 / 300, 1,168 / 728; 1280 x 256 [20] 122 / 117,
+# 603 / 394, 1,180 / 962; 1536 x 256 [24] 121 / 157, 607 / 567, 1,228 / 1,424;
+# 1024 x 1024 [64] 240 / 312, 950 / 1,128; 4096 x 1024 [256] 903 / 1,283.
+# Ragged: 602 x 256 [10] 106 / 88, 593 / 282, 1,159 / 718; 1433 x 41 [12]
+# 101 / 56, 226 / 194, 437 / 476; 511 x 509 [16] 117 / 121; 602 x 602 [25]
+# 128 / 214, 607 / 790; 8415 x 16 [66] 139 / 257, 558 / 987.
 F32_TN_ROWS = 16384
+F32_TN_TILES = 20
+F32_TN_RAGGED = 10
 
 
 def _spmm_timed(graph, x: torch.Tensor, residual: torch.Tensor = None):
@@ -67,16 +79,23 @@ def _autocast_operand(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+def _f32_tn_pays(x: torch.Tensor, g: torch.Tensor) -> bool:
+    """Whether x^T @ g has few enough output tiles for the split-K f32 kernel."""
+    whole = all(t.shape[1] % 4 == 0 and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (x, g))
+    return _ops.gemm_tn_f32_tiles(x.shape[1], g.shape[1]) <= (F32_TN_TILES if whole else F32_TN_RAGGED)
+
+
 def _weight_grad(x: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     """x^T @ g: the split-K gfx950 kernel for tall f16/bf16 operands (the
     library GEMM leaves most of the chip idle on this shape), torch
-    otherwise.  float32 result from the kernel.  Tall f32 operands take the
-    f32 kernel, except where autocast would multiply them in 16 bits and in
-    a backward that is itself recorded (create_graph)."""
+    otherwise.  float32 result from the kernel.  Tall f32 operands of a small
+    product (_f32_tn_pays) take the f32 kernel, except where autocast would
+    multiply them in 16 bits and in a backward that is itself recorded
+    (create_graph)."""
     if x.shape[0] >= 4096 and _ops.gemm_tn_supported(x, g):
         return _ops.gemm_tn(x, g, out_dtype=torch.float32)
-    if (x.shape[0] >= F32_TN_ROWS and _ops.gemm_tn_f32_supported(x, g) and not torch.is_grad_enabled()
-            and not torch.is_autocast_enabled("cuda")):
+    if (x.shape[0] >= F32_TN_ROWS and _ops.gemm_tn_f32_supported(x, g) and _f32_tn_pays(x, g)
+            and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")):
         return _ops.gemm_tn_f32(x, g)
     return torch.matmul(x.t(), g)
 

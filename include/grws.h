@@ -727,8 +727,10 @@ size_t grws_gemm_tn_workspace_bytes(int64_t K, int64_t M, int64_t N);
 int grws_gemm_tn(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t in_dtype, int64_t K,
                  int64_t M, int64_t N, void* c, int64_t ldc, int32_t out_dtype, void* workspace,
                  size_t workspace_bytes, void* stream);
-/* The same product of F32 operands (F32 matrix instructions, F32 partials); */
-/* any widths and row strides (whole 16-byte rows load faster).              */
+/* The same product of F32 operands (F32 matrix instructions, F32 partials): */
+/* widths of at most 65,536, row strides of at least the width (whole        */
+/* 16-byte rows load faster).  At least 8 partials of M x N, unless K has    */
+/* fewer than 8 x 256 rows: meant for small outputs of a long K.             */
 size_t grws_gemm_tn_f32_workspace_bytes(int64_t K, int64_t M, int64_t N);
 int grws_gemm_tn_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int64_t K, int64_t M,
                      int64_t N, float* c, int64_t ldc, void* workspace, size_t workspace_bytes,

@@ -1,9 +1,11 @@
 """Host-side layout rules of the ops layer (no device work): line-pitched
 buffers, the paired-product layout and the rule that decides when the
 convolution adds its self term inside the SpMM."""
+import pytest
 import torch
 
 from graph_rws_amd.core import ops
+from graph_rws_amd.layers import layer
 
 
 def test_line_pitched_empty_rows_start_on_lines():
@@ -42,3 +44,39 @@ def test_fuse_self_rule():
     assert ops.fuse_self_pays(232_965, 256, 2)
     assert not ops.fuse_self_pays(2_449_029, 256, 2)
     assert ops.fuse_self_pays(2708, 16, 4)
+
+
+@pytest.mark.parametrize("m,n,tiles", [(7, 7, 1), (32, 33, 1), (64, 128, 1), (129, 65, 2), (128, 129, 2), (1024, 256, 16),
+                                       (1433, 16, 12), (8415, 41, 66)])
+def test_f32_weight_gradient_tiles(m, n, tiles):
+    assert ops.gemm_tn_f32_tiles(m, n) == ops.gemm_tn_f32_tiles(n, m) == tiles
+
+
+# 20 tiles of whole vectors, 21; 10 ragged tiles, 11; wide on either side
+@pytest.mark.parametrize("m,n,kernel", [(128, 256, True), (7, 41, True), (2560, 32, True), (2564, 32, False),
+                                        (1280, 256, True), (1536, 256, False), (1279, 7, True), (1281, 7, False),
+                                        (602, 256, True), (602, 602, False), (16, 8415, False), (2048, 2048, False)])
+def test_f32_weight_gradient_leaves_wide_products_to_the_library(monkeypatch, m, n, kernel):
+    """The f32 split-K kernel takes products of few output tiles only: with
+    more the library is faster and needs no partial sums."""
+    monkeypatch.setattr(layer, "F32_TN_ROWS", 8)
+    monkeypatch.setattr(ops, "gemm_tn_f32_supported", lambda a, b: True)
+    monkeypatch.setattr(ops, "gemm_tn_f32", lambda a, b: "kernel")
+    x, g = torch.ones(8, m), torch.ones(8, n)
+    with torch.no_grad():
+        got = layer._weight_grad(x, g)
+    assert (isinstance(got, str) and got == "kernel") == kernel
+    if not kernel:
+        assert got.shape == (m, n) and bool((got == 8).all())
+
+
+def test_f32_weight_gradient_counts_misaligned_rows_as_ragged(monkeypatch):
+    monkeypatch.setattr(layer, "F32_TN_ROWS", 8)
+    monkeypatch.setattr(ops, "gemm_tn_f32_supported", lambda a, b: True)
+    monkeypatch.setattr(ops, "gemm_tn_f32", lambda a, b: "kernel")
+    wide = torch.ones(8, 2560 + 8)
+    g = torch.ones(8, 16)
+    with torch.no_grad():
+        assert isinstance(layer._weight_grad(wide[:, :2560], g), str)       # 20 tiles, whole vectors
+        assert torch.is_tensor(layer._weight_grad(wide[:, 1:2561], g))      # a start 4 bytes off
+        assert torch.is_tensor(layer._weight_grad(torch.ones(8, 2562)[:, :2560], g))  # a pitch of 2,562

@@ -1676,7 +1676,21 @@ static int sample_blocks_impl(const int64_t* indptr, const int32_t* indices, int
     }
     // A hop's transpose is a chain of ~10 small dependent kernels (45 us of a
     // 1,024-seed batch's 258 us); on the device's second stream it runs beside
-    // the next hops' sampling.  Without a next hop it stays on the caller's.
+    // the next hops' sampling, when the next hop has kBesideEdges edge slots to
+    // sample.  Below, the batch takes as long as the host's ~60 launches, and
+    // a fork and its join add events to them.  When the next hop is the last
+    // and transposed too, its chain soon waits for the side stream (they share
+    // the sort's buffers): kBesideEdgesLast.  Batches, us, on the caller's
+    // stream / every transpose on the second one / by this rule: fanouts
+    // 15,10,5, layers 1 and 2 transposed, 1 seed 288 / 300 / 278, 256 seeds 333 /
+    // 318 / 300, 1,024 seeds 400 / 362 / 364, 8,192 seeds 816 / 638 / 634; 10,5, both
+    // transposed, 1 seed 230 / 255 / 222, 1,024 seeds 291 / 300 / 288, 8,192 seeds
+    // 491 / 470 / 480.
+    constexpr int64_t kBesideEdges = 32768, kBesideEdgesLast = 131072;
+    auto beside = [&](int h) {
+        if (h + 1 >= H) return false;
+        return c.E[h + 1] >= (h + 2 == H && thops[h + 1] ? kBesideEdgesLast : kBesideEdges);
+    };
     SideStream ss(stream);
     for (int h = 0; h < H; ++h) {
         const int k = fanouts[h];
@@ -1711,10 +1725,11 @@ static int sample_blocks_impl(const int64_t* indptr, const int32_t* indices, int
 #undef GRWS_MH_WINDOWS
         GRWS_LAUNCH_CHECK();
         if (any_t && thops[h]) {
-            // the hop's slots are still in the workspace: its transposed block
-            // (once forked, every later transpose follows on the side stream:
-            // they share the sort's buffers)
-            if (h + 1 < H || ss.side != ss.main) GRWS_TRY(ss.fork_again());
+            // the hop's slots are still in the workspace: its transposed block.
+            // One on the caller's stream first waits for those on the side
+            // stream (they share the sort's buffers)
+            if (beside(h)) GRWS_TRY(ss.fork_again());
+            else GRWS_TRY(ss.join());
             const hipStream_t tstream = ss.side;
             const int64_t ecap = c.E[h], wcap = c.WT[h];
 #define GRWS_MH_T(KERNEL, VT, ...) hipLaunchKernelGGL(KERNEL<VT>, __VA_ARGS__)

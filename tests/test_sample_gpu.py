@@ -234,6 +234,11 @@ def _tensor_np(t: torch.Tensor) -> np.ndarray:
 @pytest.mark.parametrize("hops,tc,vdt,mask", [([5, 10, 15], 16, torch.float32, None),
                                               ([5, 10, 15], 8, torch.float16, None),
                                               ([5, 10, 15], 16, torch.bfloat16, [True, False, True]),
+                                              # 36,000 and 117,000 edge slots in the later hops: both
+                                              # transposes on the second stream; 312,000 in the last: the
+                                              # middle one there, then the last on the caller's
+                                              ([5, 20, 15], 16, torch.float16, [True, True, False]),
+                                              ([5, 10, 40], 8, torch.float32, [True, True, True]),
                                               ([64, 1], 16, torch.float32, None),
                                               ([2] * 8, 16, torch.float16, None)])
 def test_sample_blocks_transposed_bit_exact(cuda_device, hops, tc, vdt, mask):

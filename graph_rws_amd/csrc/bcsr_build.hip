@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kBlk = 256;
 
-enum : int32_t { kErrRow = kErrEdgeRow, kErrCol = kErrEdgeCol, kErrRowPtr = 4 };
+enum : int32_t { kErrRow = kErrEdgeRow, kErrCol = kErrEdgeCol, kErrRowPtr = 4, kErrCount = 8 };
 
 // Bits needed to hold every value in [0, x).
 inline int bits_for(int64_t x) {
@@ -1221,7 +1221,12 @@ __global__ __launch_bounds__(256) void tile_window_kernel(const int64_t* __restr
 // consecutive tiles, so its edges take consecutive places from its first
 // tile's toff: they are packed in LDS and written by consecutive lanes (each
 // lane storing its own few edges took 24 store instructions for ~50 edges a
-// wave: 1.85 ms for 114.6M edges in 16x16 f16 tiles).
+// wave: 1.85 ms for 114.6M edges in 16x16 f16 tiles).  With KEYS a wave
+// writes the places that toff gives its tiles and no others, and all nnz
+// places are written and none past them, whatever the caller's count was: one
+// that is not toff's total, or tiles that hold another number of edges than
+// was counted, is flagged in err, and the places left over get the key 0 (an
+// edge of the first window): the sort sees no key that was never written.
 template <typename VT, bool ALIGNED, bool KEYS>
 __global__ __launch_bounds__(256) void tile_emit_kernel(const int32_t* __restrict__ twin,
                                                         const int32_t* __restrict__ cols,
@@ -1230,19 +1235,24 @@ __global__ __launch_bounds__(256) void tile_emit_kernel(const int32_t* __restric
                                                         int32_t* __restrict__ out_rows,
                                                         int32_t* __restrict__ out_cols,
                                                         float* __restrict__ out_vals, int cbits, int wbits,
-                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ pay) {
+                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ pay,
+                                                        int64_t nnz, int32_t* __restrict__ err) {
     constexpr int V = 16 / (int)sizeof(VT);
     constexpr int CAP = 64 * V;  // edges of a wave's chunks
     __shared__ uint64_t srcd[4][CAP];  // row << 32 | column
     __shared__ float sval[4][CAP];
-    const int tpb = 16 * tc / V;
-    const int64_t nch = T * tpb;
+    const int tsh = __builtin_ctz(16 * tc / V);  // 16 tc / V chunks a tile, a power of two
+    const int64_t nch = T << tsh;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     for (int64_t xb = (int64_t)blockIdx.x * 256 + wave * kWave; xb < nch; xb += (int64_t)gridDim.x * 256) {
         const int64_t x = xb + lane;
         const bool in = x < nch;
-        const int64_t t = in ? x / tpb : 0;
-        const int s0 = in ? (int)(x % tpb) * V : 0;
+        const int64_t t = in ? x >> tsh : 0;
+        const int s0 = in ? ((int)x & ((1 << tsh) - 1)) * V : 0;
+        // the counted edges of the wave's tiles take places base .. base + room - 1
+        const int64_t base = toff[xb >> tsh];
+        int64_t room = 0;
+        if constexpr (KEYS) room = toff[(xb + kWave < nch ? xb + kWave : nch) >> tsh] - base;
         float v[V];
         int32_t cc[V];
         uint32_t ok = 0;
@@ -1278,8 +1288,17 @@ __global__ __launch_bounds__(256) void tile_emit_kernel(const int32_t* __restric
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int64_t base = toff[xb / tpb];
-        for (int i = lane; i < total; i += kWave) {
+        int n = total;
+        if constexpr (KEYS) {
+            if (lane == 0 && room != total) atomicOr(err, kErrCount);
+            if (room > nnz - base) room = nnz - base;
+            for (int64_t i = total + lane; i < room; i += kWave) {
+                keys[base + i] = 0;
+                pay[base + i] = 0u;
+            }
+            n = room < total ? (int)room : total;
+        }
+        for (int i = lane; i < n; i += kWave) {
             const uint64_t rc = srcd[wave][i];
             const int64_t r = (int64_t)(rc >> 32), cl = (int64_t)(uint32_t)rc;
             if constexpr (KEYS) {
@@ -1294,6 +1313,14 @@ __global__ __launch_bounds__(256) void tile_emit_kernel(const int32_t* __restric
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if constexpr (KEYS) {
+        const int64_t counted = toff[T];
+        if (counted != nnz && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, kErrCount);
+        for (int64_t i = counted + (int64_t)blockIdx.x * 256 + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * 256) {
+            keys[i] = 0;
+            pay[i] = 0u;
+        }
     }
 }
 
@@ -1344,6 +1371,7 @@ int report_input_error(int32_t e, const char* who) {
     if (e & kErrRowPtr) return set_error(GRWS_E_RANGE, "%s: row_ptr is not a valid CSR row pointer", who);
     if (e & kErrRow) return set_error(GRWS_E_RANGE, "%s: a row index is out of range", who);
     if (e & kErrCol) return set_error(GRWS_E_RANGE, "%s: a column index is out of range", who);
+    if (e & kErrCount) return set_error(GRWS_E_RANGE, "%s: nnz is not the count of the graph's edges", who);
     return GRWS_OK;
 }
 
@@ -1741,7 +1769,7 @@ static int launch_tile_windows(const grws_bcsr* A, int32_t* twin, hipStream_t st
 template <bool KEYS>
 static int launch_tile_emit(const grws_bcsr* A, int64_t num_cols, const int32_t* twin, const int64_t* toff,
                             int32_t* rows, int32_t* cols, float* values, int cbits, int wbits, uint64_t* keys,
-                            uint32_t* pay, hipStream_t stream) {
+                            uint32_t* pay, int64_t nnz, int32_t* err, hipStream_t stream) {
     const int64_t nch = A->num_tiles * 16 * A->tile_cols / (16 / dtype_size(A->values_dtype));
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((nch + 255) / 256, 65536));
     const bool al = tiles_aligned(A);
@@ -1749,11 +1777,11 @@ static int launch_tile_emit(const grws_bcsr* A, int64_t num_cols, const int32_t*
     if (al)                                                                                                        \
         hipLaunchKernelGGL((tile_emit_kernel<VT, true, KEYS>), dim3(grid), dim3(256), 0, stream, twin,             \
                            A->col_indices, A->values, A->num_tiles, A->tile_cols, num_cols, toff, rows, cols,      \
-                           values, cbits, wbits, keys, pay);                                                       \
+                           values, cbits, wbits, keys, pay, nnz, err);                                             \
     else                                                                                                           \
         hipLaunchKernelGGL((tile_emit_kernel<VT, false, KEYS>), dim3(grid), dim3(256), 0, stream, twin,            \
                            A->col_indices, A->values, A->num_tiles, A->tile_cols, num_cols, toff, rows, cols,      \
-                           values, cbits, wbits, keys, pay)
+                           values, cbits, wbits, keys, pay, nnz, err)
     switch (A->values_dtype) {
         case GRWS_F32: GRWS_TILE_EMIT(float); break;
         case GRWS_F16: GRWS_TILE_EMIT(_Float16); break;
@@ -1822,7 +1850,8 @@ extern "C" int grws_bcsr_to_coo_fill(const grws_bcsr* A, int64_t num_cols, int32
     // the count's per-tile counts are spent (toff holds their scan): the
     // array takes each tile's window
     GRWS_TRY(launch_tile_windows(A, cnt, stream));
-    GRWS_TRY(launch_tile_emit<false>(A, num_cols, cnt, toff, rows, cols, values, 0, 0, nullptr, nullptr, stream));
+    GRWS_TRY(launch_tile_emit<false>(A, num_cols, cnt, toff, rows, cols, values, 0, 0, nullptr, nullptr, 0, nullptr,
+                                     stream));
     return GRWS_OK;
 }
 
@@ -1911,16 +1940,23 @@ extern "C" int grws_bcsr_transpose_count(const grws_bcsr* A, int64_t num_cols, i
         return set_error(GRWS_E_CAPACITY, "bcsr_transpose: workspace too small (%zu < %zu)", workspace_bytes, cv.used);
     int32_t* twin = nullptr;
     int64_t* toff = nullptr;
-    if (nnz > 0) {
+    if (nnz > 0 || (A->num_tiles > 0 && coo_workspace)) {
         char* sws;
         size_t sb;
         GRWS_TRY(coo_ws(coo_workspace, coo_workspace_bytes, A->num_tiles, &twin, &toff, &sws, &sb));
+    }
+    if (nnz > 0) {
         // the per-tile counts are spent (toff holds their scan)
         GRWS_TRY(launch_tile_windows(A, twin, stream));
+    } else if (toff) {  // no keys to make: the count is compared here
+        int64_t counted = 0;
+        GRWS_HIP(hipMemcpyAsync(&counted, toff + A->num_tiles, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+        GRWS_HIP(hipStreamSynchronize(stream));
+        if (counted != 0) return report_input_error(kErrCount, "bcsr_transpose");
     }
     return build_count(nullptr, s, w, nullptr, nullptr, nullptr, nnz, rows, num_cols, tile_cols, 1, window_offset,
                        num_tiles_out, stream, [&](int wbits) -> int {
         return launch_tile_emit<true>(A, num_cols, twin, toff, nullptr, nullptr, nullptr, s.cbits, wbits, w.ka, w.va,
-                                      stream);
+                                      nnz, w.err, stream);
     });
 }

@@ -371,7 +371,9 @@ int grws_bcsr_to_coo_fill(const grws_bcsr* A, int64_t num_cols, int32_t* rows, i
  * grws_bcsr_to_coo_count (its nnz and its workspace, kept as it left it),
  * the edges go to the sort without the COO arrays between.  Same result and
  * workspace as grws_bcsr_build_count(rows, cols, values of the COO, nnz,
- * 16 * num_windows, num_cols, transpose = 1); grws_bcsr_build_fill follows. */
+ * 16 * num_windows, num_cols, transpose = 1); grws_bcsr_build_fill follows.
+ * GRWS_E_RANGE, and no graph, when nnz is not that count or the tiles hold
+ * other numbers of edges than were counted (another graph or num_cols). */
 int grws_bcsr_transpose_count(const grws_bcsr* A, int64_t num_cols, int64_t nnz, void* coo_workspace,
                               size_t coo_workspace_bytes, int32_t tile_cols, int64_t* window_offset,
                               void* workspace, size_t workspace_bytes, int64_t* num_tiles_out,

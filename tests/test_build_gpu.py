@@ -628,6 +628,46 @@ def test_transpose_keys_from_tiles_equal_the_coo_route(cuda_device, vdt, tc, off
     assert empty[0].tolist() == [0, 0, 0] and empty[1].numel() == 0 and empty[2].numel() == 0
 
 
+@pytest.mark.parametrize("vdt,tc", [(torch.float32, 8), (torch.float16, 16)])
+def test_transpose_count_refuses_another_edge_count(cuda_device, vdt, tc):
+    """An nnz that is not the counted number, and a num_cols that was not
+    counted with, are GRWS_E_RANGE; nothing is written past the workspace
+    that the given nnz asks for, and the right call still works after."""
+    import ctypes
+    from graph_rws_amd.core import _lib as L
+    g = synth.chung_lu(777, 9000, 2.1, seed=8)
+    hw, hc, hv = _host(g, tc)
+    w, c, v = hw.to(cuda_device), hc.to(cuda_device), hv.to(vdt).view(-1).to(cuda_device)
+    ncols = g.num_nodes
+
+    def call(num_cols, nnz, guard=1 << 16):
+        view, counted, cws = builder._coo_count(w, c, v, tc, ncols, "test")
+        n = counted if nnz is None else nnz(counted)
+        rows = 16 * view.num_windows
+        win = torch.empty((num_cols + 15) // 16 + 1, dtype=torch.int64, device=cuda_device)
+        wsb = int(L.load().grws_bcsr_build_workspace_bytes(n, rows, num_cols, 1))
+        ws = torch.full((wsb + guard,), 0x5a, dtype=torch.uint8, device=cuda_device)
+        T = ctypes.c_int64()
+        print(f"case transpose count nnz={n} counted={counted} num_cols={num_cols}", flush=True)
+        try:
+            L.call("grws_bcsr_transpose_count", ctypes.byref(view), num_cols, n, L.ptr(cws), cws.numel(), tc,
+                   L.ptr(win), L.ptr(ws), wsb, ctypes.byref(T), L.stream_of(cuda_device))
+        finally:
+            assert bool((ws[wsb:] == 0x5a).all())
+        return win
+
+    right = call(ncols, None)
+    for wrong in (lambda n: n - 1, lambda n: n + 1, lambda n: n // 3, lambda n: n + 700, lambda n: 1, lambda n: 0):
+        with pytest.raises(GrwsError, match="count of the graph's edges"):
+            call(ncols, wrong)
+    for cols in (ncols - 300, ncols // 2, 1):
+        with pytest.raises(GrwsError, match="count of the graph's edges"):
+            call(cols, None)
+    assert torch.equal(call(ncols, None), right)
+    win, _, _ = builder.transpose_arrays(w, c, v, tc, ncols)
+    assert torch.equal(win, right)
+
+
 class _Loaded:
     """What a graph loader hands over (num_nodes, edges, edata, device), also
     as a message-flow block."""

@@ -241,6 +241,7 @@ struct TopkShared {
     uint64_t prefix;
     int32_t shift;
     int32_t k;
+    int32_t placed, ranks;  // the direct ranking's kept candidates and the sum of their ranks
     int32_t col[kMaxCap];
     int32_t slot[kMaxCap];
     uint64_t kmin[BLK / kWave], kmax[BLK / kWave];
@@ -250,7 +251,11 @@ struct TopkShared {
 // Selects active window b's sample (its columns in ascending order and their
 // slots, -1 past the sample) and its output tile count.  Every thread of the
 // work-group calls it with the same b; it leaves LDS to the caller's next
-// window only after a barrier.
+// window only after a barrier.  A window's columns are distinct in every
+// graph built here.  One listed twice (arrays from elsewhere) counts once per
+// slot, the lower slot first, in windows of up to kTopkBlk candidates; in
+// larger ones it is unspecified which of a repeated column's slots are kept,
+// and whether they crowd out others.
 template <typename VT, int BLK, int KC, int HW>
 __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const int64_t b, const int32_t li,
                                             const TopkArgs& a) {
@@ -386,15 +391,20 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
     if (packed) nscan = count;
 
     if (cached && count <= FASTMAX) {
-        // a candidate's rank is the number of smaller keys (keys are
-        // distinct; ~0 marks a non-candidate and is above them all), the cap
-        // first are kept, and each kept one's output place is the number of
-        // kept columns below its own: two passes over LDS, no select or sort.
+        // a candidate's rank is the number of smaller keys (~0 marks a
+        // non-candidate and is above them all), the cap first are kept, and
+        // each kept one's output place is the number of kept columns below its
+        // own: two passes over LDS, no select or sort.
         // Keys past nslots read as ~0: the scan runs over whole 8-key groups
-        // in 16-byte LDS reads
+        // in 16-byte LDS reads.  Distinct keys take the ranks 0 .. nsel - 1
+        // once each; a repeated column's take lower ones (their number or sum
+        // shows it), and are then ranked again, equal keys in slot order
         const int ngrp = (int)((nslots + 7) / 8);
+        const int nsel = count < cap ? count : cap;
         for (int64_t s = nslots + tid; s < 8 * (int64_t)ngrp; s += BLK) sh.key[s] = ~0ull;
+        if (tid == 0) sh.placed = sh.ranks = 0;
         __syncthreads();
+        int placed = 0, ranks = 0;
         for (int64_t s = tid; s < nslots; s += BLK) {
             const uint64_t k = sh.key[s];
             if (k == ~0ull) continue;
@@ -408,14 +418,33 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
             if (r < cap) {
                 sh.col[r] = (int32_t)(uint32_t)k;
                 sh.slot[r] = (int32_t)s;
+                ++placed;
+                ranks += r;
             }
         }
+        if (placed) {
+            atomicAdd(&sh.placed, placed);
+            atomicAdd(&sh.ranks, ranks);
+        }
         __syncthreads();
-        const int nsel = count < cap ? count : cap;
+        if (sh.placed != nsel || sh.ranks != nsel * (nsel - 1) / 2) {  // uniform over the work-group
+            for (int64_t s = tid; s < nslots; s += BLK) {
+                const uint64_t k = sh.key[s];
+                if (k == ~0ull) continue;
+                int r = 0;
+                for (int64_t j = 0; j < nslots; ++j) r += sh.key[j] < k || (sh.key[j] == k && j < s) ? 1 : 0;
+                if (r < cap) {
+                    sh.col[r] = (int32_t)(uint32_t)k;
+                    sh.slot[r] = (int32_t)s;
+                }
+            }
+            __syncthreads();
+        }
         for (int i = tid; i < nsel; i += BLK) {
             const int32_t c = sh.col[i];
             int pos = 0;
-            for (int j = 0; j < nsel; ++j) pos += sh.col[j] < c ? 1 : 0;
+            for (int j = 0; j < nsel; ++j)
+                pos += sh.col[j] < c || (sh.col[j] == c && sh.slot[j] < sh.slot[i]) ? 1 : 0;
             if (pos < S) {
                 oc[pos] = c;
                 os[pos] = sh.slot[i];
@@ -431,7 +460,7 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
     }
     {
         static_assert(BLK >= kMaxCap, "the bitonic sort takes one thread per entry");
-        // radix select of the cap-th smallest key (keys are distinct)
+        // radix select of the cap-th smallest key
         uint64_t prefix = 0;
         int shift = 64;  // selected: key >> shift <= prefix >> shift (shift 64: all)
         if (count > cap) {
@@ -757,7 +786,7 @@ __device__ __forceinline__ void topk_wave_window(const TopkArgs& a, int64_t b, i
         for (int i = lane; i < nsel; i += kWave) {
             const int32_t c = scol[i];
             int pos = 0;
-            for (int j = 0; j < nsel; ++j) pos += scol[j] < c ? 1 : 0;
+            for (int j = 0; j < nsel; ++j) pos += scol[j] < c || (scol[j] == c && j < i) ? 1 : 0;
             if (pos < S) {
                 oc[pos] = c;
                 os[pos] = sslot[i];

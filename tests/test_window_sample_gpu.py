@@ -370,3 +370,77 @@ def test_count_nonzero_matches_torch(cuda_device, dt):
     arrays += [base[i:i + 50] for i in range(40)]
     got = ops.count_nonzero(arrays)
     assert got.tolist() == [int(torch.count_nonzero(a)) for a in arrays]
+
+
+def _listed_windows(slots, tc, rng, most=None, holes=0.1):
+    """A BCSR of one window per entry of `slots` (multiples of tc): distinct
+    columns in permuted order, some slots empty, at most `most` columns, and
+    values of few magnitudes, so that many columns have equal scores."""
+    win = np.concatenate([[0], np.cumsum(np.asarray(slots) // tc)]).astype(np.int64)
+    cols = np.full(int(win[-1]) * tc, -1, np.int32)
+    for i, n in enumerate(slots):
+        at = rng.permutation(n)[:min(n - int(holes * n), most or n)]
+        cols[int(win[i]) * tc + at] = rng.permutation(40000)[:at.size]
+    T = int(win[-1])
+    vals = (rng.integers(0, 3, (T, 16, tc)) * (rng.random((T, 16, tc)) < 0.2) * 0.25).astype(np.float32)
+    vals[np.broadcast_to((cols.reshape(T, 1, tc) == -1), vals.shape)] = 0
+    return win, cols, vals
+
+
+# slots around what a lane of the one-wave kernel holds (4, 8 and 16 x 64),
+# and windows of the big kernel: keys in LDS, more than that
+_SLOTS = {8: [8, 248, 256, 264, 504, 512, 520, 1016, 1024, 1032, 2048, 4096, 4104, 9000],
+          16: [16, 240, 256, 272, 496, 512, 528, 1008, 1024, 1040, 2064, 4096, 4112, 9008]}
+
+
+@pytest.mark.parametrize("tc", [8, 16])
+@pytest.mark.parametrize("fanout", [3, 40, 200, 256])
+def test_windows_in_any_column_order(cuda_device, tc, fanout):
+    """Windows whose columns are listed in any order, with empty slots
+    between, bit for bit against the oracle at every edge of the kernels'
+    sizes (the builders list columns ascending)."""
+    print(f"case permuted windows tc={tc} fanout={fanout}", flush=True)
+    rng = np.random.default_rng(100 * tc + fanout)
+    slots = _SLOTS[tc] + [n for n in _SLOTS[tc] if n < 600]
+    win, cols, vals = _listed_windows(slots, tc, rng)
+    seeds = np.arange(len(slots)) * 16 + 3
+    got, _ = sample_all_layers(torch.from_numpy(win).to(cuda_device), torch.from_numpy(cols).to(cuda_device),
+                               torch.from_numpy(vals).view(-1).to(cuda_device),
+                               torch.from_numpy(seeds).to(cuda_device), [fanout], 40000, tile_cols=tc)
+    _compare(got, oracle.window_sample_all_layers(win, cols, vals.reshape(-1), seeds, [fanout], 40000, tile_cols=tc))
+
+
+@pytest.mark.parametrize("tc", [8, 16])
+@pytest.mark.parametrize("fanout", [3, 40, 200])
+@pytest.mark.parametrize("order", ["ascending", "permuted"])
+def test_windows_listing_a_column_more_than_once(cuda_device, tc, fanout, order):
+    """A repeated column counts once per slot, the lower slot first: the
+    sample of the graph whose occurrences are renamed apart, 64 c + occurrence,
+    in windows of up to 1,024 candidates (the one-wave kernel's and the big
+    kernel's direct ranking), with repeats on both sides of the cut."""
+    print(f"case repeated columns tc={tc} fanout={fanout} {order}", flush=True)
+    rng = np.random.default_rng(7 * tc + fanout)
+    slots = [n for n in _SLOTS[tc] if n <= 4096]
+    win, cols, vals = _listed_windows(slots, tc, rng, most=1000)
+    apart = cols.astype(np.int64)
+    for i in range(len(slots)):
+        a, b = int(win[i]) * tc, int(win[i + 1]) * tc
+        c = cols[a:b]
+        used = np.flatnonzero(c >= 0)
+        c[used] = rng.integers(0, max(2, used.size // 3), used.size)  # each about three times
+        if order == "ascending":
+            c[used] = np.sort(c[used])
+        seen = {}
+        for j in used:
+            k = seen[c[j]] = seen.get(c[j], -1) + 1
+            apart[a + j] = 64 * int(c[j]) + k
+        assert max(seen.values(), default=0) < 64
+    if tc == 8 and fanout == 3:
+        vals[vals != 0] = 0.5  # scores by the number of nonzeros only: many whole keys equal
+    seeds = np.arange(len(slots)) * 16 + 3
+    args = [torch.from_numpy(x).to(cuda_device) for x in (win, cols, vals.reshape(-1), seeds)]
+    got, _ = sample_all_layers(*args[:3], args[3], [fanout], 40000, tile_cols=tc)
+    want = oracle.window_sample_all_layers(win, apart.astype(np.int32), vals.reshape(-1), seeds, [fanout], 64 * 40000,
+                                           tile_cols=tc)
+    want[0][1] = np.where(want[0][1] >= 0, want[0][1] // 64, -1).astype(np.int32)
+    _compare(got, want)

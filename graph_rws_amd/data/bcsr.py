@@ -26,11 +26,17 @@ import torch
 from ..core import csr_to_bcsr_cpu, build_spmm_plan, default_slabs
 
 
-# Longest window (slabs) that a sampled block's product takes in one work item.
-# Such a graph is multiplied once, and a plan costs it 15 launches and a
-# stream sync (190 us of a 1,024-seed mini-batch step, for one 40-slab
-# window); a wave walks a slab in well under 1 us.
+# A sampled block of windows up to SAMPLED_SLABS slabs is multiplied without a
+# plan, each window as one work item, until its products have walked
+# PLAN_SLABS slabs more than a plan's items would, one after another in their
+# longest window: it is mostly multiplied once, and building a plan takes 15
+# launches and a stream sync, 160 us, what 200 slabs take in f32 (0.8 us each;
+# 0.15-0.5 in 16 bits).  Measured, one product of 1,500 windows with 16 of h
+# slabs, 608 f32 columns (us, without / with a plan, plus 160 to build it):
+# h = 32 65 / 45, h = 64 102 / 49, h = 128 179 / 55, h = 256 337 / 67, where the
+# plan pays at once; 128 bf16 columns: h = 128 38 / 13.
 SAMPLED_SLABS = 128
+PLAN_SLABS = 200
 
 
 def _placed(t: torch.Tensor, device, dtype: torch.dtype) -> torch.Tensor:
@@ -294,20 +300,30 @@ class BCSRGraph:
         schedule and no plan needs building.  A graph whose arrays are
         refilled in place between replays of a captured step
         (``refilled = True``) never takes a plan: its windows change under
-        the plan."""
+        the plan.  A sampled block takes one once its products have shown
+        that it is kept (PLAN_SLABS), never while a stream is captured (a
+        build synchronises)."""
         if getattr(self, "refilled", False):
             return None
         slabs = default_slabs(self.num_windows, self.num_tiles, self.tile_cols, n_cols)
         mws = getattr(self, "max_window_slabs", None)
-        if mws is not None and (mws <= slabs or (mws <= SAMPLED_SLABS and getattr(self, "sampled", False))):
+        if mws is not None and mws <= slabs:
             return None
         from ..core.ops import TensorKey
+        state = ((self.window_offset,), (self.num_tiles, self.tile_cols))
         ent = self._cache.get(("plan", slabs))
-        if ent is None or not ent[0].matches((self.window_offset,), (self.num_tiles, self.tile_cols)):
-            p = build_spmm_plan(self.window_offset, self.num_tiles, self.tile_cols, slabs)
-            ent = (TensorKey((self.window_offset,), (self.num_tiles, self.tile_cols)), p)
-            self._cache[("plan", slabs)] = ent
-        return ent[1]
+        if ent is not None and ent[0].matches(*state):
+            return ent[1]
+        if mws is not None and mws <= SAMPLED_SLABS and getattr(self, "sampled", False):
+            walked = self._cache.get(("walked", slabs))
+            if walked is None or not walked[0].matches(*state):
+                walked = self._cache[("walked", slabs)] = [TensorKey(*state), 0]
+            if walked[1] <= PLAN_SLABS or torch.cuda.is_current_stream_capturing():
+                walked[1] += mws - slabs
+                return None
+        p = build_spmm_plan(self.window_offset, self.num_tiles, self.tile_cols, slabs)
+        self._cache[("plan", slabs)] = (TensorKey(*state), p)
+        return p
 
     def packed_tiles(self):
         """The packed copy of the values the SpMM reads instead of the dense

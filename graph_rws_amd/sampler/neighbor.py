@@ -144,7 +144,7 @@ class NeighborSampler:
             # at most 16 x fanout distinct columns per window
             g.max_window_slabs = (16 * k + 15) // 16
             g.fanout = k
-            g.sampled = True  # multiplied in one step, then dropped
+            g.sampled = True  # mostly multiplied in one step, then dropped
             if tr is not None:
                 from ..core.ops import TensorKey
                 twin, tcols, tvals, tmax = tr

@@ -80,3 +80,56 @@ def test_f32_weight_gradient_counts_misaligned_rows_as_ragged(monkeypatch):
         assert isinstance(layer._weight_grad(wide[:, :2560], g), str)       # 20 tiles, whole vectors
         assert torch.is_tensor(layer._weight_grad(wide[:, 1:2561], g))      # a start 4 bytes off
         assert torch.is_tensor(layer._weight_grad(torch.ones(8, 2562)[:, :2560], g))  # a pitch of 2,562
+
+
+def _windows(slabs, max_slabs, sampled):
+    """A BCSR (host arrays) of short windows and one of `slabs` 16-column slabs."""
+    from graph_rws_amd.data import BCSRGraph
+    tiles = torch.tensor([1, slabs, 2, 1])
+    win = torch.cat([torch.zeros(1, dtype=torch.int64), tiles.cumsum(0)])
+    T = int(win[-1])
+    g = BCSRGraph(num_nodes=64, num_edges=0, tile_rows=16, tile_cols=16, window_offset=win,
+                  original_col_indices=torch.zeros(16 * T, dtype=torch.int32),
+                  values_condensed=torch.zeros(256 * T), device="cpu", num_rows=64, num_cols=5000)
+    g.max_window_slabs = max_slabs
+    if sampled:
+        g.sampled = True
+    return g
+
+
+# (longest window, products before the first with a plan): none needed up to a
+# plan's own item (16 slabs); 200 slabs walked in excess; past 128 at once
+@pytest.mark.parametrize("slabs,before", [(16, None), (17, 201), (40, 9), (128, 2), (129, 0), (400, 0)])
+def test_sampled_block_takes_a_plan_when_it_is_kept(monkeypatch, slabs, before):
+    from graph_rws_amd.data import bcsr
+    built = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(bcsr, "build_spmm_plan", lambda *a, **k: built.append(1) or "plan")
+    g = _windows(slabs, slabs, True)
+    assert ops.default_slabs(g.num_windows, g.num_tiles, 16, 128) == 16
+    if before is None:
+        assert all(g.spmm_plan(128) is None for _ in range(300)) and not built
+        return
+    for i in range(before):
+        assert g.spmm_plan(128) is None, i
+    assert g.spmm_plan(128) == "plan" and g.spmm_plan(128) == "plan" and built == [1]
+    # other windows in the same buffer: the count starts again
+    g.window_offset.add_(0)
+    if before:
+        assert g.spmm_plan(128) is None
+    # not sampled, or of unknown windows: at the first product
+    assert _windows(slabs, slabs, False).spmm_plan(128) == "plan"
+    assert _windows(slabs, None, True).spmm_plan(128) == "plan"
+
+
+def test_sampled_block_builds_no_plan_under_capture(monkeypatch):
+    from graph_rws_amd.data import bcsr
+    monkeypatch.setattr(bcsr, "build_spmm_plan", lambda *a, **k: "plan")
+    capturing = [True]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    g = _windows(128, 128, True)
+    assert all(g.spmm_plan(64) is None for _ in range(5))
+    capturing[0] = False
+    assert g.spmm_plan(64) == "plan"
+    capturing[0] = True
+    assert g.spmm_plan(64) == "plan"  # built before the capture: used in it

@@ -313,3 +313,48 @@ def test_neighbor_sampler_blocks_carry_their_transposes(cuda_device):
         assert AT.max_window_slabs == fresh.max_window_slabs
         G = torch.randn(16 * b.num_windows, 32, device=cuda_device).half()
         torch.testing.assert_close(AT.spmm(G), fresh.spmm(G), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("seeds,plan_at", [(640, 9), (2000, 2), (4096, 0)])
+def test_kept_sampled_block_with_a_hub_window(cuda_device, seeds, plan_at):
+    """The transpose of a block whose seeds share one neighbour has a window
+    of 40, 125 or 256 slabs: the product number plan_at is the first that
+    takes a plan, and every product, one replayed from a graph captured
+    before that among them, matches 64 bits: sums of at most `seeds` f32
+    terms, in any order."""
+    from graph_rws_amd import builder
+    n = 3 * seeds
+    print(f"case hub transpose seeds={seeds}", flush=True)
+    indptr = torch.arange(n + 1, dtype=torch.int64, device=cuda_device)
+    indices = torch.full((n,), n - 1, dtype=torch.int32, device=cuda_device)  # every node's neighbour is the last
+    s = NeighborSampler([1], tile_cols=16)
+    block, = s.sample_layers(indptr, indices, torch.arange(seeds, device=cuda_device), transposes=[True])
+    AT = block.transpose()
+    assert AT.max_window_slabs == seeds // 16
+    rows, cols, vals = builder.bcsr_to_coo(AT.window_offset, AT.original_col_indices, AT.values_condensed, 16,
+                                           AT.num_cols)
+    G = torch.randn(16 * block.num_windows, 128, device=cuda_device)
+    terms = vals.double()[:, None] * G.double()[cols.long()]
+    ref = torch.zeros(16 * AT.num_windows, 128, dtype=torch.float64, device=cuda_device)
+    size = ref.index_add(0, rows.long(), terms.abs())
+    ref.index_add_(0, rows.long(), terms)
+
+    def check(Y):
+        assert bool(((Y.double() - ref).abs() <= (seeds + 1) * 2.0 ** -24 * size).all())
+
+    out = None
+    if plan_at:
+        check(AT.spmm(G))
+        stream = torch.cuda.Stream(cuda_device)
+        graph = torch.cuda.CUDAGraph()
+        stream.wait_stream(torch.cuda.current_stream(cuda_device))
+        with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+            out = AT.spmm(G)
+    assert ("plan", 16) not in AT._cache
+    for i in range(2 if plan_at else 0, plan_at + 2):
+        check(AT.spmm(G))
+        assert (("plan", 16) in AT._cache) == (i >= plan_at), i
+        if out is not None:
+            graph.replay()
+            torch.cuda.synchronize()
+            check(out)

@@ -4,7 +4,7 @@ the same f16/bf16 inputs.  Bound: |C - C64| <= 1e-4 * (|A|^T |B|) elementwise
 import pytest
 import torch
 
-from graph_rws_amd.core.ops import gemm_tn, gemm_tn_f32, gemm_tn_supported
+from graph_rws_amd.core.ops import gemm_tn, gemm_tn_f32, gemm_tn_f32_tiles, gemm_tn_supported
 
 pytestmark = pytest.mark.gpu
 
@@ -96,9 +96,9 @@ def test_graphconv_autocast_backward_uses_split_k(cuda_device):
                                    (9000, 1433, 16), (100003, 128, 256), (65536, 200, 41)])
 def test_gemm_tn_f32_matches_float64(cuda_device, K, M, N):
     """Edges of the 32/64/128-column tiles, ragged widths and K
-    remainders.  Bound: a chunk of k rows summed in f32 in order, then the
-    chunks' partials: (k + chunks) * 2^-24 of |A|^T |B|; chunks have at most
-    max(256, K tiles / 512) + 32 rows, under 8,192 here."""
+    remainders.  Bound: a chunk's rows summed in f32 in order, then the
+    chunks' partials: (rows + chunks) * 2^-24 of |A|^T |B|, with the split's
+    own chunks (f32_shape in csrc/gemm_tn.hip)."""
     g = torch.Generator(device=cuda_device).manual_seed(K + M + N)
     A = torch.randn(K, M, generator=g, device=cuda_device)
     B = torch.randn(K, N, generator=g, device=cuda_device)
@@ -106,7 +106,9 @@ def test_gemm_tn_f32_matches_float64(cuda_device, K, M, N):
     assert C.shape == (M, N) and C.dtype == torch.float32
     ref = A.double().t() @ B.double()
     bound = A.double().abs().t() @ B.double().abs()
-    assert bool(((C.double() - ref).abs() <= (8192 + 512) * 2.0 ** -24 * bound + 1e-30).all())
+    chunks = max(1, min(max(8, 512 // gemm_tn_f32_tiles(M, N) // 8 * 8), -(-K // 256)))
+    rows = -(-(-(-K // chunks)) // 32) * 32
+    assert bool(((C.double() - ref).abs() <= (rows + chunks) * 2.0 ** -24 * bound).all())
     assert torch.equal(C, gemm_tn_f32(A, B))  # deterministic
     wide = torch.full((K, N + 9), float("nan"), device=cuda_device)
     wide[:, :N] = B  # a column view of a wider buffer: its padding must not reach the result
@@ -115,14 +117,35 @@ def test_gemm_tn_f32_matches_float64(cuda_device, K, M, N):
     assert torch.equal(C, gemm_tn_f32(A, wide[:, 1:N + 1]))
 
 
+@pytest.mark.parametrize("K,M,N", [(1, 4, 4), (31, 32, 36), (33, 64, 65), (255, 33, 64), (257, 65, 7), (4097, 64, 129),
+                                   (9001, 1433, 16), (16387, 24, 9), (65537, 200, 41), (100003, 128, 256)])
+@pytest.mark.parametrize("wide", ["a", "b"])
+def test_gemm_tn_f32_is_exact_on_integers(cuda_device, K, M, N, wide):
+    """One operand of odd integers below 4,096 (12 bits: more than an f16 or
+    bf16 holds), the other of -1 and 1: every partial sum is a whole number
+    below 2^24 (a random walk of 100,003 steps of 2,400 ends under 7.6e5 in
+    its root mean square, the limit is 22 times that), so f32 adds exactly
+    in any order, and an operand rounded to 16 bits, a row lost from a
+    remainder or one taken twice shows in the result."""
+    print(f"case gemm_tn_f32 integers K={K} M={M} N={N} {wide}", flush=True)
+    g = torch.Generator(device=cuda_device).manual_seed(3 * K + M + N)
+    big = [M, N][wide == "b"]
+    W = torch.randint(0, 2048, (K, big), generator=g, device=cuda_device) * 2 + 1
+    W = (W * (torch.randint(0, 2, (K, big), generator=g, device=cuda_device) * 2 - 1)).float()
+    S = (torch.randint(0, 2, (K, M + N - big), generator=g, device=cuda_device) * 2 - 1).float()
+    A, B = (W, S) if wide == "a" else (S, W)
+    assert torch.equal(gemm_tn_f32(A, B).double(), A.double().t() @ B.double())
+
+
 def test_tall_f32_weight_grad_of_expanded_and_batched_operands(cuda_device):
     """Operands the f32 kernel does not take (rows that share memory,
-    gradients batched by vmap) go to the library's product."""
+    gradients batched by vmap) go to the library's product.  Whole numbers
+    up to 8: every sum is below 2^24, so the product is exact."""
     from graph_rws_amd.layers.layer import F32_TN_ROWS, _weight_grad
     n = F32_TN_ROWS + 3
     gen = torch.Generator(device=cuda_device).manual_seed(5)
-    x = torch.randn(n, 24, generator=gen, device=cuda_device)
-    g = torch.randn(n, 9, generator=gen, device=cuda_device)
+    x = torch.randint(1, 9, (n, 24), generator=gen, device=cuda_device).float()
+    g = torch.randint(1, 9, (n, 9), generator=gen, device=cuda_device).float()
     ones = torch.ones(1, 24, device=cuda_device).expand(n, 24)
 
     class Product(torch.autograd.Function):
@@ -135,15 +158,14 @@ def test_tall_f32_weight_grad_of_expanded_and_batched_operands(cuda_device):
         def backward(ctx, grad):
             return None, _weight_grad(ctx.saved_tensors[0], grad.contiguous())
 
-    def close(c, a, b):  # n f32 sums
-        bound = a.double().abs().t() @ b.double().abs()
-        assert bool(((c.double() - a.double().t() @ b.double()).abs() <= n * 2.0 ** -24 * bound).all())
+    def same(c, a, b):
+        assert torch.equal(c.double(), a.double().t() @ b.double())
 
     with torch.no_grad():
-        close(_weight_grad(ones, g), ones, g)
-        close(_weight_grad(x, g), x, g)
+        same(_weight_grad(ones, g), ones, g)
+        same(_weight_grad(x, g), x, g)
     w = torch.randn(24, 9, generator=gen, device=cuda_device, requires_grad=True)
     both = torch.stack([g, 2 * g])
     dw, = torch.autograd.grad(Product.apply(x, w), w, both, is_grads_batched=True)
-    close(dw[0], x, g)
-    close(dw[1], x, 2 * g)
+    same(dw[0], x, g)
+    same(dw[1], x, 2 * g)

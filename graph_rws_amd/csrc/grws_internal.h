@@ -276,9 +276,6 @@ int scan_i32_to_i64(const int32_t* in, int64_t* out, int64_t n, bool inclusive, 
 int scan_i64_to_i64(const int64_t* in, int64_t* out, int64_t n, bool inclusive, void* ws,
                     size_t ws_bytes, hipStream_t stream);
 
-// Stable LSD radix sort of (u64 key, u32 payload) pairs over the low `bits`
-// key bits (sort.hip).  The result lands in keys/vals or, when
-// *result_in_alt, in keys_alt/vals_alt.
 // An edge list as the window-major sort reads it: ids (int32, or int64 taken
 // modulo 2^32), f32 values (NULL: 1.0), and where bad ids are flagged.
 enum : int32_t { kErrEdgeRow = 1, kErrEdgeCol = 2 };
@@ -299,14 +296,18 @@ __device__ __forceinline__ uint64_t window_key(int64_t wr, int64_t cc, int wbits
     return (uint64_t)(wr >> 4) | ((uint64_t)(wr & 15) << wbits) | ((uint64_t)cc << (wbits + 4));
 }
 
+// Stable LSD radix sort of (u64 key, u32 payload) pairs over the low `bits`
+// key bits (sort.hip).  The result lands in keys/vals or, when
+// *result_in_alt, in keys_alt/vals_alt.
 size_t radix_sort_workspace_bytes(int64_t n);
-// The pairs sort of an edge list's window-major keys over their low `bits`
-// bits; the first pass makes the keys (radix_sorts_edges(n) says whether).
+int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits,
+                     void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt);
+// The same sort of an edge list's window-major keys: the first pass makes the
+// keys from `coo` and does not read keys/vals.  Only where
+// radix_sorts_edges(n), and bits > 0.
 bool radix_sorts_edges(int64_t n);
 int radix_sort_edges(const CooEdges& coo, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                      int64_t n, int bits, void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt);
-int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits,
-                     void* ws, size_t ws_bytes, hipStream_t stream, bool* result_in_alt);
 
 // Fill helpers (plain kernels: safe under graph capture, unlike memset nodes).
 int fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t stream);

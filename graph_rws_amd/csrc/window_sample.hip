@@ -29,12 +29,13 @@
 //     column j (or -1) and its tile_rows values are that column's values in
 //     the input window (or 0), :520-578.
 //
-// Design: one work-group per active window (256 threads up to 1,024 slots,
-// 1,024 threads beyond, those windows' keys computed beforehand by many
-// work-groups).  The 64-bit key (~total << 32 | column) orders candidates
-// exactly as the reference's comparator; up to 1,024 candidates are ranked
-// directly, more go through an MSB-first 8-bit radix select (passes start at
-// the first byte where the candidates' keys differ) that finds the CAP-th
+// Design: one wave per active window of up to 1,024 slots, its keys in
+// registers, the CAP-th smallest found bit by bit; one work-group of 1,024
+// threads for a larger one, its keys computed beforehand by many work-groups.
+// The 64-bit key (~total << 32 | column) orders candidates exactly as the
+// reference's comparator; in a larger window up to 1,024 candidates are
+// ranked directly, more go through an MSB-first 8-bit radix select (passes
+// start at the first byte where the candidates' keys differ) that finds the CAP-th
 // key, and the selected (column, slot) pairs are compacted into LDS and
 // bitonic-sorted by column.  The slot index replaces the reference's linear
 // column search when the tiles are rebuilt.  Every layer of a batch can run

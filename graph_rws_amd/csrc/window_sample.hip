@@ -242,9 +242,14 @@ struct TopkShared {
     uint64_t prefix;
     int32_t shift;
     int32_t k;
-    int32_t placed, ranks;  // the direct ranking's kept candidates and the sum of their ranks
-    int32_t col[kMaxCap];
-    int32_t slot[kMaxCap];
+    int32_t repeat;  // the direct ranking met a column listed twice
+    union {
+        struct {
+            int32_t col[kMaxCap];
+            int32_t slot[kMaxCap];
+        };
+        uint64_t pair[kMaxCap];  // the direct ranking's: column (sign flipped) << 32 | slot
+    };
     uint64_t kmin[BLK / kWave], kmax[BLK / kWave];
     __attribute__((aligned(16))) uint64_t key[KC + 8];
 };
@@ -394,18 +399,21 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
     if (cached && count <= FASTMAX) {
         // a candidate's rank is the number of smaller keys (~0 marks a
         // non-candidate and is above them all), the cap first are kept, and
-        // each kept one's output place is the number of kept columns below its
-        // own: two passes over LDS, no select or sort.
+        // each kept one's output place is the number of kept (column, slot)
+        // pairs below its own: two passes over LDS, no select or sort.
         // Keys past nslots read as ~0: the scan runs over whole 8-key groups
-        // in 16-byte LDS reads.  Distinct keys take the ranks 0 .. nsel - 1
-        // once each; a repeated column's take lower ones (their number or sum
-        // shows it), and are then ranked again, equal keys in slot order
+        // in 16-byte LDS reads.  Distinct keys fill the places 0 .. nsel - 1;
+        // equal ones (a repeated column) meet in one, the lowest slot stays,
+        // and an empty place says that the rest have to be ranked by slot
         const int ngrp = (int)((nslots + 7) / 8);
         const int nsel = count < cap ? count : cap;
         for (int64_t s = nslots + tid; s < 8 * (int64_t)ngrp; s += BLK) sh.key[s] = ~0ull;
-        if (tid == 0) sh.placed = sh.ranks = 0;
+        if (tid < kMaxCap) sh.pair[tid] = ~0ull;
+        if (tid == 0) sh.repeat = 0;
         __syncthreads();
-        int placed = 0, ranks = 0;
+        auto pair_of = [](uint64_t k, int64_t s) {
+            return (uint64_t)((uint32_t)k ^ 0x80000000u) << 32 | (uint32_t)s;
+        };
         for (int64_t s = tid; s < nslots; s += BLK) {
             const uint64_t k = sh.key[s];
             if (k == ~0ull) continue;
@@ -416,39 +424,28 @@ __device__ __forceinline__ void topk_window(TopkShared<BLK, KC, HW>& sh, const i
                 r += (k0.x < k) + (k0.y < k) + (k1.x < k) + (k1.y < k) + (k2.x < k) + (k2.y < k) + (k3.x < k) +
                      (k3.y < k);
             }
-            if (r < cap) {
-                sh.col[r] = (int32_t)(uint32_t)k;
-                sh.slot[r] = (int32_t)s;
-                ++placed;
-                ranks += r;
-            }
-        }
-        if (placed) {
-            atomicAdd(&sh.placed, placed);
-            atomicAdd(&sh.ranks, ranks);
+            if (r < cap) atomicMin((unsigned long long*)&sh.pair[r], (unsigned long long)pair_of(k, s));
         }
         __syncthreads();
-        if (sh.placed != nsel || sh.ranks != nsel * (nsel - 1) / 2) {  // uniform over the work-group
+        if (tid < nsel && sh.pair[tid] == ~0ull) sh.repeat = 1;
+        __syncthreads();
+        if (sh.repeat) {  // uniform over the work-group
             for (int64_t s = tid; s < nslots; s += BLK) {
                 const uint64_t k = sh.key[s];
                 if (k == ~0ull) continue;
                 int r = 0;
                 for (int64_t j = 0; j < nslots; ++j) r += sh.key[j] < k || (sh.key[j] == k && j < s) ? 1 : 0;
-                if (r < cap) {
-                    sh.col[r] = (int32_t)(uint32_t)k;
-                    sh.slot[r] = (int32_t)s;
-                }
+                if (r < cap) sh.pair[r] = pair_of(k, s);
             }
             __syncthreads();
         }
         for (int i = tid; i < nsel; i += BLK) {
-            const int32_t c = sh.col[i];
+            const uint64_t c = sh.pair[i];
             int pos = 0;
-            for (int j = 0; j < nsel; ++j)
-                pos += sh.col[j] < c || (sh.col[j] == c && sh.slot[j] < sh.slot[i]) ? 1 : 0;
+            for (int j = 0; j < nsel; ++j) pos += sh.pair[j] < c ? 1 : 0;
             if (pos < S) {
-                oc[pos] = c;
-                os[pos] = sh.slot[i];
+                oc[pos] = (int32_t)((uint32_t)(c >> 32) ^ 0x80000000u);
+                os[pos] = (int32_t)(uint32_t)c;
             }
         }
         for (int i = nsel + tid; i < S; i += BLK) {
